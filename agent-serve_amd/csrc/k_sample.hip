@@ -10,12 +10,27 @@
 //      `last` and z (the same sum, so the same float), p_i /= z for i < last;
 //   5. the first i whose running sum reaches the draw r, else the last kept index.
 //
-// Steps 2 and the divisions run on every thread; the running sums (3-5) are sequential
-// float additions in the reference, so one wave performs them in order from registers
-// (64 values per load, eight loads ahead), one lane-broadcast addition per element. A sum
-// stops early once the next value is at most a quarter of an ulp of the sum: the values
-// do not increase, so none of the rest can change it (sharp distributions stop after a
-// handful of elements; a nearly flat one over a 128K vocabulary takes the whole pass).
+// The running sums (3-5) are sequential float additions in the reference, so one wave performs
+// them in order from registers (64 values per load, eight loads ahead), one lane-broadcast
+// addition per element. A sum stops early once the next value is at most a quarter of an ulp
+// of the sum: the values do not increase, so none of the rest can change it (sharp
+// distributions stop after a handful of elements; a nearly flat one over a 128K vocabulary
+// takes the whole pass).
+//
+// Two ways to the same token:
+//   launch_sample_top   only the logits with (l_i - max) / T >= -20 are picked out and sorted
+//                       (in LDS, at most kTopCap of them). The others have p_i < 2^-28, below a
+//                       quarter ulp of every sum they would be added to (s >= 1, and the sums
+//                       of p_i / s end within 2^-11 of 1), so they change nothing; only the
+//                       very last index of the order is needed besides (a draw above a sum that
+//                       stays below it takes it). Bound by its three launches and one
+//                       workgroup's sort: 38 us of kernels for a 128,256-entry vocabulary with
+//                       about 300 logits that count, where sorting everything took 530 us.
+//   launch_sample       the whole order, where more than kTopCap logits count (flat
+//                       distributions), where a logit is NaN or the maximum infinite, or where
+//                       the caller asks for the order or the probabilities.
+#include <algorithm>
+
 #include "dev_common.hpp"
 #include "expf_libm.hpp"
 #include "tf_internal.hpp"
@@ -67,27 +82,39 @@ __global__ __launch_bounds__(kBlock) void k_rs_hist(const uint32_t* key, int n, 
         for (int d = lane; d < 256; d += kWave) hist[(size_t)d * tiles + tile] = cnt[wv][d];
 }
 
-// Exclusive prefix sum of m counts in place (one workgroup).
+// Exclusive prefix sum of m counts (a multiple of 4) in place, one workgroup: segments of 4096
+// counts, a uint4 per thread (coalesced; a contiguous run per thread instead, read one word
+// at a time, took 57 us for 32,256 counts), the next segment loading while this one is summed.
 __global__ __launch_bounds__(1024) void k_rs_scan(uint32_t* hist, int m) {
-    __shared__ uint32_t part[1024];
-    const int t = threadIdx.x;
-    const int per = (m + 1023) / 1024;
-    const int b = t * per, e = min(m, b + per);
-    uint32_t sum = 0;
-    for (int i = b; i < e; ++i) sum += hist[i];
-    part[t] = sum;
-    __syncthreads();
-    for (int o = 1; o < 1024; o <<= 1) {
-        const uint32_t v = t >= o ? part[t - o] : 0u;
+    __shared__ uint32_t wsum[2][16];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    uint4* h4 = (uint4*)hist;
+    const int n4 = m / 4;
+    const uint4 zero = make_uint4(0, 0, 0, 0);
+    uint32_t base = 0;
+    uint4 cur = t < n4 ? h4[t] : zero;
+    for (int i0 = 0, it = 0; i0 < n4; i0 += 1024, it ^= 1) {
+        const int i = i0 + t;
+        const uint4 nxt = i + 1024 < n4 ? h4[i + 1024] : zero;
+        const uint32_t sum = cur.x + cur.y + cur.z + cur.w;
+        uint32_t inc = sum;  // inclusive scan over the wave
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t v = (uint32_t)__shfl_up((int)inc, o);
+            inc += lane >= o ? v : 0u;
+        }
+        if (lane == 63) wsum[it][wave] = inc;
         __syncthreads();
-        part[t] += v;
-        __syncthreads();
-    }
-    uint32_t run = part[t] - sum;
-    for (int i = b; i < e; ++i) {
-        const uint32_t c = hist[i];
-        hist[i] = run;
-        run += c;
+        uint32_t before = 0, all = 0;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) {
+            before += w < wave ? wsum[it][w] : 0u;
+            all += wsum[it][w];
+        }
+        const uint32_t r = base + before + inc - sum;
+        if (i < n4) h4[i] = make_uint4(r, r + cur.x, r + cur.x + cur.y, r + cur.x + cur.y + cur.z);
+        base += all;
+        cur = nxt;
     }
 }
 
@@ -128,130 +155,241 @@ __device__ __forceinline__ float quarter_ulp(float s) {
     return (__uint_as_float(__float_as_uint(s) + 1u) - s) * 0.25f;
 }
 
-// Wave 0's view of p[0..n): 64 values per register, eight registers per refill, the next
-// eight loading while these are consumed.
-struct Seq {
-    const float* p;
-    int n, lane;
+__device__ __forceinline__ float lane_value(float v, int j) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
+}
+
+// Calls f(i, value) for i = 0, 1, ... over val(0), val(1), ... val(n - 1) in order, one wave:
+// 64 values per register, eight registers per refill, the next eight loading while these
+// are consumed. `stuck(first)` ends it before a group of 64 whose first (largest) value
+// can no longer change the sum; f ends it by returning true.
+template <class Val, class Stuck, class F>
+__device__ __forceinline__ void in_order(int n, Val val, Stuck stuck, F f) {
+    const int lane = threadIdx.x & 63;
     float cur[8], nxt[8];
-    __device__ void load(int base, float (&b)[8]) {
+    auto load = [&](int base, float (&b)[8]) {
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
             const int i = base + 64 * c + lane;
-            b[c] = i < n ? p[i] : 0.0f;
+            b[c] = i < n ? val(i) : 0.0f;
+        }
+    };
+    load(0, cur);
+    for (int base = 0; base < n; base += 512) {
+        load(base + 512, nxt);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const int cb = base + 64 * c;
+            if (cb < n) {
+                if (stuck(lane_value(cur[c], 0))) return;
+                const int cnt = min(64, n - cb);
+                for (int j = 0; j < cnt; ++j)
+                    if (f(cb + j, lane_value(cur[c], j))) return;
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 8; ++c) cur[c] = nxt[c];
+    }
+}
+
+// Steps 3-5 on one wave over p_0 .. p_(n-1) in descending order (the values before any
+// division; a division by s or z is the same float wherever it happens). Returns the place
+// picked, or -1 for the last kept one; `total` is the place count of the whole order,
+// which `last` reads when the nucleus takes everything.
+struct Picked {
+    int place, last;
+    float s, z;
+};
+__device__ __forceinline__ Picked pick(const float* p, int n, int total, float top_p, float r) {
+    Picked o{-1, total, 0.0f, 0.0f};
+    float s = 0.0f;
+    in_order(n, [&](int i) { return p[i]; }, [&](float v) { return v <= quarter_ulp(s); },
+             [&](int, float v) {
+                 s += v;
+                 return false;
+             });
+    float acc = 0.0f;
+    if (top_p < 1.0f)
+        in_order(n, [&](int i) { return p[i] / s; }, [&](float v) { return v <= quarter_ulp(acc); },
+                 [&](int i, float v) {
+                     acc += v;
+                     if (acc >= top_p) {
+                         o.last = i + 1;
+                         return true;
+                     }
+                     return false;
+                 });
+    const float z = acc;
+    o.s = s;
+    o.z = z;
+    acc = 0.0f;
+    in_order(min(n, o.last), [&](int i) { return top_p < 1.0f ? p[i] / s / z : p[i] / s; },
+             [&](float v) { return v <= quarter_ulp(acc); },
+             [&](int i, float v) {
+                 acc += v;
+                 if (r <= acc) {
+                     o.place = i;
+                     return true;
+                 }
+                 return false;
+             });
+    return o;
+}
+
+// Step 2 for the whole order.
+__global__ __launch_bounds__(kBlock) void k_sample_exp(const float* logits, const int32_t* idx, float* p, int n,
+                                                       float temperature) {
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    const float m = logits[idx[0]];
+    if (i < n) p[i] = expf_libm((logits[idx[i]] - m) / temperature, kExp2Tab);
+}
+
+// Steps 3-5 for the whole order (one workgroup): the token and, for a caller that asked,
+// the final probabilities in place of p.
+__global__ __launch_bounds__(kSampleThreads) void k_sample(const int32_t* idx, float* p, int n, float top_p, float r,
+                                                           int32_t* out, int want_probs) {
+    __shared__ Picked sh;
+    if (threadIdx.x < 64) {
+        const Picked o = pick(p, n, n, top_p, r);
+        if (threadIdx.x == 0) {
+            *out = idx[o.place >= 0 ? o.place : o.last - 1];
+            sh = o;
         }
     }
+    if (!want_probs) return;
+    __syncthreads();
+    const Picked o = sh;
+    for (int i = threadIdx.x; i < n; i += kSampleThreads) {
+        const float v = p[i] / o.s;
+        p[i] = top_p < 1.0f && i < o.last ? v / o.z : v;
+    }
+}
+
+// ---- the logits that count only (launch_sample_top)
+
+constexpr int kTopCap = 4096;      // entries the LDS sort holds
+constexpr int kTopBlocks = 64;     // workgroups of the two passes over the logits
+constexpr float kTopCut = -20.0f;  // e^-20 < 2^-28
+
+// Scratch: the passes' results, then the picked (key, index) entries.
+struct TopWork {
+    unsigned long long hi[kTopBlocks];  // per workgroup: least (key, index), the largest logit
+    unsigned long long lo[kTopBlocks];  // greatest (key, index), the last of the order
+    int32_t nan[kTopBlocks];            // a NaN among its logits
+    int32_t count;                      // entries picked (may exceed kTopCap)
+    unsigned long long list[kTopCap];
 };
 
-// Steps 2-5 for the logits in the order idx (one workgroup).
-__global__ __launch_bounds__(kSampleThreads) void k_sample(const float* logits, const int32_t* idx, float* p, int n,
-                                                           float temperature, float top_p, float r, int32_t* out) {
-    __shared__ float sh_s, sh_z;
-    __shared__ int sh_last;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const bool w0 = tid < 64;
-    const float m = logits[idx[0]];
-    for (int i = tid; i < n; i += kSampleThreads) p[i] = expf_libm((logits[idx[i]] - m) / temperature, kExp2Tab);
-    __syncthreads();
-    Seq q{p, n, lane};
-    // 3: s in order
-    if (w0) {
-        float s = 0.0f;
-        q.load(0, q.cur);
-        for (int base = 0; base < n; base += 512) {
-            q.load(base + 512, q.nxt);
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const int cb = base + 64 * c;
-                if (cb < n) {
-                    if (__int_as_float(__builtin_amdgcn_readlane(__float_as_int(q.cur[c]), 0)) <= quarter_ulp(s))
-                        goto s_done;
-                    const int cnt = min(64, n - cb);
-                    for (int j = 0; j < cnt; ++j) s += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q.cur[c]), j));
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < 8; ++c) q.cur[c] = q.nxt[c];
-        }
-    s_done:
-        if (lane == 0) sh_s = s;
+__device__ __forceinline__ unsigned long long top_entry(float l, int i) {
+    return ((unsigned long long)desc_key(l) << 32) | (uint32_t)i;
+}
+
+// Pass 1: each workgroup's first and last entry of the order.
+__global__ __launch_bounds__(kBlock) void k_top_range(const float* logits, int n, TopWork* w) {
+    __shared__ unsigned long long sh_hi[kWavesPerBlock], sh_lo[kWavesPerBlock];
+    __shared__ int sh_nan[kWavesPerBlock];
+    unsigned long long hi = ~0ull, lo = 0ull;
+    int nan = 0;
+    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += kTopBlocks * kBlock) {
+        const float l = logits[i];
+        const unsigned long long e = top_entry(l, i);
+        hi = e < hi ? e : hi;
+        lo = e > lo ? e : lo;
+        nan |= l != l;
+    }
+    hi = ~wave_max_u64(~hi);
+    lo = wave_max_u64(lo);
+    nan = __ballot(nan) != 0ull;
+    const int wave = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+        sh_hi[wave] = hi;
+        sh_lo[wave] = lo;
+        sh_nan[wave] = nan;
     }
     __syncthreads();
-    const float s = sh_s;
-    for (int i = tid; i < n; i += kSampleThreads) p[i] = p[i] / s;
-    __syncthreads();
-    // 4: nucleus
-    if (w0) {
-        int last = n;
-        float acc = 0.0f;
-        if (top_p < 1.0f) {
-            q.load(0, q.cur);
-            for (int base = 0; base < n; base += 512) {
-                q.load(base + 512, q.nxt);
-#pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    const int cb = base + 64 * c;
-                    if (cb < n) {
-                        // stuck below top_p: the sum never reaches it, every value stays
-                        if (__int_as_float(__builtin_amdgcn_readlane(__float_as_int(q.cur[c]), 0)) <= quarter_ulp(acc))
-                            goto p_done;
-                        const int cnt = min(64, n - cb);
-                        for (int j = 0; j < cnt; ++j) {
-                            acc += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q.cur[c]), j));
-                            if (acc >= top_p) {
-                                last = cb + j + 1;
-                                goto p_done;
-                            }
-                        }
-                    }
-                }
-#pragma unroll
-                for (int c = 0; c < 8; ++c) q.cur[c] = q.nxt[c];
-            }
+    if (threadIdx.x == 0) {
+        for (int k = 1; k < kWavesPerBlock; ++k) {
+            hi = sh_hi[k] < hi ? sh_hi[k] : hi;
+            lo = sh_lo[k] > lo ? sh_lo[k] : lo;
+            nan |= sh_nan[k];
         }
-    p_done:
-        if (lane == 0) {
-            sh_last = last;
-            sh_z = acc;
-        }
+        w->hi[blockIdx.x] = hi;
+        w->lo[blockIdx.x] = lo;
+        w->nan[blockIdx.x] = nan;
+        if (blockIdx.x == 0) w->count = 0;
     }
+}
+
+// The largest logit: lane b of every wave reads workgroup b's entry (kTopBlocks is a wave).
+__device__ __forceinline__ float top_max(const float* logits, const TopWork* w) {
+    static_assert(kTopBlocks == kWave, "a lane per workgroup of the first pass");
+    return logits[(uint32_t)~wave_max_u64(~w->hi[threadIdx.x & 63])];
+}
+
+// Pass 2: the entries that count, in any order (the sort makes it one), a place per wave and
+// round from one atomic.
+__global__ __launch_bounds__(kBlock) void k_top_pick(const float* logits, int n, float temperature, TopWork* w) {
+    const float m = top_max(logits, w);
+    const int lane = threadIdx.x & 63;
+    for (int i0 = blockIdx.x * kBlock + (threadIdx.x & ~63); i0 < n; i0 += kTopBlocks * kBlock) {
+        const int i = i0 + lane;
+        const float l = i < n ? logits[i] : 0.0f;
+        const bool in = i < n && (l - m) / temperature >= kTopCut;
+        const uint64_t mask = __ballot(in);
+        if (!mask) continue;
+        int base = 0;
+        if (lane == 0) base = atomicAdd(&w->count, __popcll(mask));
+        base = __builtin_amdgcn_readfirstlane(base) + __popcll(mask & ((1ull << lane) - 1ull));
+        if (in && base < kTopCap) w->list[base] = top_entry(l, i);
+    }
+}
+
+// Sort, probabilities and the pick, one workgroup. *out < 0: the whole order is needed.
+__global__ __launch_bounds__(kSampleThreads) void k_top_sample(const float* logits, int n, float temperature,
+                                                               float top_p, float r, const TopWork* w, int32_t* out) {
+    __shared__ unsigned long long e[kTopCap];
+    __shared__ float p[kTopCap];
+    const int tid = threadIdx.x, count = w->count;
+    const float m = top_max(logits, w);
+    const bool nan = __ballot(w->nan[tid & 63] != 0) != 0ull;
+    if (nan || !(fabsf(m) < INFINITY) || count > kTopCap || count < 1) {
+        if (tid == 0) *out = -1;
+        return;
+    }
+    int size = 64;  // the power of two that holds the entries
+    while (size < count) size *= 2;
+    for (int i = tid; i < size; i += kSampleThreads) e[i] = i < count ? w->list[i] : ~0ull;
     __syncthreads();
-    const int last = sh_last;
-    if (top_p < 1.0f) {
-        const float z = sh_z;
-        for (int i = tid; i < last; i += kSampleThreads) p[i] = p[i] / z;
-        __syncthreads();
-    }
-    // 5: the draw
-    if (w0) {
-        int tok = idx[last - 1];
-        float acc = 0.0f;
-        Seq f{p, last, lane};
-        f.load(0, f.cur);
-        for (int base = 0; base < last; base += 512) {
-            f.load(base + 512, f.nxt);
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const int cb = base + 64 * c;
-                if (cb < last) {
-                    // stuck below r: no later element is picked
-                    if (__int_as_float(__builtin_amdgcn_readlane(__float_as_int(f.cur[c]), 0)) <= quarter_ulp(acc))
-                        goto r_done;
-                    const int cnt = min(64, last - cb);
-                    for (int j = 0; j < cnt; ++j) {
-                        acc += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f.cur[c]), j));
-                        if (r <= acc) {
-                            tok = idx[cb + j];
-                            goto r_done;
-                        }
-                    }
+    // bitonic sort, thread t taking pair t (entries 2 t - (t mod j) and + j). A step with
+    // j <= 64 stays inside the 128 entries of each wave's pairs, so between two such steps the
+    // wave's own LDS order is enough (36 of the 55 steps for 1024 entries)
+    for (int k = 2; k <= size; k *= 2)
+        for (int j = k / 2; j > 0; j /= 2) {
+            for (int t = tid; t < size / 2; t += kSampleThreads) {
+                const int a = 2 * t - (t & (j - 1)), b = a + j;
+                const unsigned long long x = e[a], y = e[b];
+                if ((x > y) == ((a & k) == 0)) {
+                    e[a] = y;
+                    e[b] = x;
                 }
             }
-#pragma unroll
-            for (int c = 0; c < 8; ++c) f.cur[c] = f.nxt[c];
+            if (j > 64 || (j == 1 && k > 64)) {  // the next step's distance is j / 2, or k after j = 1
+                __syncthreads();
+            } else {
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
         }
-    r_done:
-        if (lane == 0) *out = tok;
+    __syncthreads();
+    for (int i = tid; i < count; i += kSampleThreads)
+        p[i] = expf_libm((logits[(uint32_t)e[i]] - m) / temperature, kExp2Tab);
+    __syncthreads();
+    if (tid < 64) {
+        const Picked o = pick(p, count, n, top_p, r);
+        const int at = o.place >= 0 ? o.place : o.last - 1;
+        // a draw past every sum: the last kept index, the whole order's last one if all are kept
+        const unsigned long long lo = wave_max_u64(w->lo[tid]);
+        if (tid == 0) *out = (int32_t)(uint32_t)(at < count ? e[at] : lo);
     }
 }
 
@@ -260,7 +398,17 @@ __global__ __launch_bounds__(kSampleThreads) void k_sample(const float* logits, 
 size_t sample_work_bytes(int n) {
     const size_t a = ((size_t)n * 4 + 255) / 256 * 256;
     const size_t tiles = ((size_t)n + kRsTile - 1) / kRsTile;
-    return 5 * a + (256 * tiles * 4 + 255) / 256 * 256;
+    return std::max(5 * a + (256 * tiles * 4 + 255) / 256 * 256, sizeof(TopWork));
+}
+
+hipError_t launch_sample_top(const float* logits, int n, float temperature, float top_p, float r, void* work,
+                             size_t work_bytes, int32_t* d_token, hipStream_t st) {
+    if (work_bytes < sizeof(TopWork)) return hipErrorInvalidValue;
+    TopWork* w = (TopWork*)work;
+    hipLaunchKernelGGL(k_top_range, dim3(kTopBlocks), dim3(kBlock), 0, st, logits, n, w);
+    hipLaunchKernelGGL(k_top_pick, dim3(kTopBlocks), dim3(kBlock), 0, st, logits, n, temperature, w);
+    hipLaunchKernelGGL(k_top_sample, dim3(1), dim3(kSampleThreads), 0, st, logits, n, temperature, top_p, r, w, d_token);
+    return hipGetLastError();
 }
 
 hipError_t launch_sample(const float* logits, int n, float temperature, float top_p, float r, void* work,
@@ -288,8 +436,10 @@ hipError_t launch_sample(const float* logits, int n, float temperature, float to
         hipError_t e = hipMemcpyAsync(d_sorted_idx, idx, (size_t)n * 4, hipMemcpyDeviceToDevice, st);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(k_sample, dim3(1), dim3(kSampleThreads), 0, st, logits, idx, p, n, temperature, top_p, r,
-                       d_token);
+    hipLaunchKernelGGL(k_sample_exp, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, logits, idx, p, n,
+                       temperature);
+    hipLaunchKernelGGL(k_sample, dim3(1), dim3(kSampleThreads), 0, st, idx, p, n, top_p, r, d_token,
+                       d_probs ? 1 : 0);
     return hipGetLastError();
 }
 

@@ -1675,11 +1675,17 @@ int tf_hip_sample(tf_hip_ctx* c, float temperature, float top_p, float r, int32_
         HIPCHK(c, hipStreamSynchronize(c->st));
         tok = key_to_index(h.key);
     } else {
-        HIPCHK(c, launch_sample(c->logits, V, temperature, top_p, r, c->sample_work, c->sample_bytes, c->d_sampled,
-                                nullptr, nullptr, c->st));
-        HIPCHK(c, hipMemcpyAsync(c->tok_host, c->d_sampled, 4, hipMemcpyDeviceToHost, c->st));
-        HIPCHK(c, hipStreamSynchronize(c->st));
-        tok = c->tok_host[0];
+        // from the logits that can matter, or from all of them where those are too many
+        for (int whole = 0; whole < 2; ++whole) {
+            HIPCHK(c, whole ? launch_sample(c->logits, V, temperature, top_p, r, c->sample_work, c->sample_bytes,
+                                            c->d_sampled, nullptr, nullptr, c->st)
+                            : launch_sample_top(c->logits, V, temperature, top_p, r, c->sample_work, c->sample_bytes,
+                                                c->d_sampled, c->st));
+            HIPCHK(c, hipMemcpyAsync(c->tok_host, c->d_sampled, 4, hipMemcpyDeviceToHost, c->st));
+            HIPCHK(c, hipStreamSynchronize(c->st));
+            tok = c->tok_host[0];
+            if (tok >= 0) break;
+        }
     }
     *token = tok;
     return 0;
@@ -1703,6 +1709,14 @@ int tf_hip_sample_logits(int device, const float* logits, int32_t n, float tempe
     if (sorted_idx) OPCHK(s.alloc(&di, (size_t)n * 4));
     if (probs) OPCHK(s.alloc(&dp, (size_t)n * 4));
     OPCHK(hipMemcpy(dl, logits, (size_t)n * 4, hipMemcpyHostToDevice));
+    int32_t tok = -1;
+    if (!sorted_idx && !probs) {
+        OPCHK(launch_sample_top(dl, n, temperature, top_p, r, work, bytes, dt, s.st));
+        OPCHK(hipMemcpyAsync(&tok, dt, 4, hipMemcpyDeviceToHost, s.st));
+        OPCHK(hipStreamSynchronize(s.st));
+        *token = tok;
+        if (tok >= 0) return 0;
+    }
     OPCHK(launch_sample(dl, n, temperature, top_p, r, work, bytes, dt, di, dp, s.st));
     OPCHK(hipMemcpyAsync(token, dt, 4, hipMemcpyDeviceToHost, s.st));
     if (sorted_idx) OPCHK(hipMemcpyAsync(sorted_idx, di, (size_t)n * 4, hipMemcpyDeviceToHost, s.st));

@@ -272,6 +272,9 @@ hipError_t launch_rmsnorm_rows(const float* x, const float* w, int n, int rows, 
 size_t sample_work_bytes(int n);
 hipError_t launch_sample(const float* logits, int n, float temperature, float top_p, float r, void* work,
                          size_t work_bytes, int32_t* d_token, int32_t* d_sorted_idx, float* d_probs, hipStream_t st);
+// The same token from the few logits that can matter; *d_token < 0 when it takes launch_sample.
+hipError_t launch_sample_top(const float* logits, int n, float temperature, float top_p, float r, void* work,
+                             size_t work_bytes, int32_t* d_token, hipStream_t st);
 hipError_t launch_rope_rows(float* x, int seq, int n_heads, int hd, int pos0, const float* cos_tab,
                             const float* sin_tab, hipStream_t st);
 hipError_t launch_argmax(const float* x, int n, Ctl* ctl, hipStream_t st);

@@ -65,6 +65,28 @@ def test_sample_logits_matches_oracle(pkg, n, scale, temp, top_p):
         assert tok == want, (k, r)
 
 
+@pytest.mark.parametrize("near", [1, 2, 63, 64, 65, 127, 128, 129, 2049, 4095, 4096, 4097])
+@pytest.mark.parametrize("rest", [-25.0, -float("inf")])
+def test_sample_few_logits_that_count(pkg, near, rest):
+    """`near` logits within 19.9 temperatures of the maximum, the rest at least 25 below it (or
+    masked to -inf): the sampler that sorts only what can change a sum (up to 4096 logits) and
+    the one that sorts everything take the oracle's token for every draw."""
+    n, temp = 20011, 0.8
+    rng = np.random.default_rng(near)
+    x = np.full(n, rest, np.float32)
+    if np.isfinite(rest):
+        x = (temp * (rest - 10.0 * rng.random(n))).astype(np.float32)
+    at = rng.permutation(n)[:near]
+    x[at] = temp * -np.linspace(0.0, 19.9, near).astype(np.float32)
+    r_hi = float(np.nextafter(np.float32(1), np.float32(0)))
+    for top_p in (1.0, 0.95, 0.3):
+        for r in [0.0, r_hi] + [float(v) for v in draws(near, 4)]:
+            want, widx, _, wlast = oracle_sample(x, temp, top_p, r)
+            if want == widx[wlast - 1] and not np.isfinite(x[want]):
+                want = n - 1 if n - 1 not in at else int(np.max(np.setdiff1d(np.arange(n), at)))  # equal logits: by index
+            assert pkg.sample_logits(x, temp, top_p, r) == want, (top_p, r)
+
+
 def test_sample_edges(pkg):
     """Draw 0 takes the most likely token, a draw just below 1 the last of the nucleus;
     temperature 0 is the first maximum; two tokens in closed form (3/4, 1/4)."""
