@@ -3,9 +3,9 @@
 //
 // k_pf_split     rmsnorm (layers.cpp:7-12) of each row, or the row as it is, scaled by
 //                a power of two and written as fp16 hi + lo in fragment order (the A operand)
-// k_pf_gemm_tile / k_pf_gemm_big   matmul (matmul.cpp:64-73) of Q8_0, Q4_0, Q4_1 or F16
-//                weights, read in their HBM layout, on v_mfma_f32_16x16x32_f16 (k_pf_gemm_q6k:
-//                Q6_K; k_pf_gemm_f32: F32 weights on v_mfma_f32_16x16x4_f32); epilogues:
+// k_pf_gemm_tile / k_pf_gemm_big   matmul (matmul.cpp:64-73) of Q8_0, Q4_0, Q4_1, F16 or
+//                Q6_K weights, read in their HBM layout, on v_mfma_f32_16x16x32_f16 (Q6_K's as
+//                fp16 pairs; k_pf_gemm_f32: F32 weights on v_mfma_f32_16x16x4_f32); epilogues:
 //                store (+ F32 bias, model.cpp:85-89), residual add (add_inplace,
 //                layers.cpp:21-23), silu(gate) * up (layers.cpp:14-19)
 // k_pf_rope_store apply_rope_many of q and k (attention.cpp:48-53) and KVCache::store
@@ -83,6 +83,7 @@ __device__ __forceinline__ h8_t q4_to_h8(uint2 w, int hi) {
 //   kSub    LDS bytes of a 16-row subtile's block (k_pf_gemm_big)
 //   kScale  bytes of one row's block in the s stream (0: no scales)
 //   kMin    Q4_1's min term
+//   kPair   the weights enter as fp16 pairs (Q6_K), with a second byte stream of kBytes2 a block
 //   off(c)  byte offset in a row's block of the piece lane c = l / 16 reads
 //   lds(p, r, c)  that piece of subtile row r from the subtile's LDS block at p
 //   cvt(raw, c)   its 8 values as fp16
@@ -93,6 +94,7 @@ struct PfW;
 template <>
 struct PfW<TF_HIP_TYPE_Q8_0> {
     static constexpr int kBytes = 32, kSub = 512, kScale = 2;
+    static constexpr bool kPair = false;
     static constexpr bool kMin = false;
     typedef uint2 Raw;
     __device__ static int off(int c) { return 8 * c; }
@@ -108,6 +110,7 @@ struct PfW<TF_HIP_TYPE_Q8_0> {
 template <>
 struct PfW<TF_HIP_TYPE_Q4_0> {
     static constexpr int kBytes = 16, kSub = 256, kScale = 2;
+    static constexpr bool kPair = false;
     static constexpr bool kMin = false;
     typedef uint2 Raw;
     __device__ static int off(int c) { return 8 * (c & 1); }
@@ -120,6 +123,7 @@ struct PfW<TF_HIP_TYPE_Q4_0> {
 template <>
 struct PfW<TF_HIP_TYPE_Q4_1> {
     static constexpr int kBytes = 16, kSub = 256, kScale = 4;
+    static constexpr bool kPair = false;
     static constexpr bool kMin = true;
     typedef uint2 Raw;
     __device__ static int off(int c) { return 8 * (c & 1); }
@@ -132,12 +136,50 @@ struct PfW<TF_HIP_TYPE_Q4_1> {
 template <>
 struct PfW<TF_HIP_TYPE_F16> {
     static constexpr int kBytes = 64, kSub = 1024, kScale = 0;
+    static constexpr bool kPair = false;
     static constexpr bool kMin = false;
     typedef uint4 Raw;
     __device__ static int off(int c) { return 16 * c; }
     __device__ static Raw load(const TF_GLOBAL uint8_t* p) { return gload_u4((const void*)p); }
     __device__ static Raw lds(const unsigned char* p, int r, int c) { return *(const uint4*)(p + 256 * c + 16 * r); }
     __device__ static h8_t cvt(Raw w, int) { return __builtin_bit_cast(h8_t, w); }
+};
+
+// Q6_K (quant.cpp:101-127). A 32-element block of a row: lo[16] in the q stream (element e < 16
+// in the low nibble of byte e, e + 16 in its high nibble), hi[8] in the q2 stream (element e's
+// top two bits at bits 2 (e / 8) of byte e % 8), two int8 scales in the s stream (one per 16
+// elements) and in s2 an fp16 d per 256: the value d sc (u - 32) for the 6-bit code u. Lane l's 8
+// elements 8 c .. 8 c + 7 share the scale sc of sub-block c / 2, folded into the operand:
+// sc (u - 32), an integer of at most 4096 in magnitude, is the fp16 pair hi (its rounding,
+// v_pk_mul_f16) + lo (the exact remainder, at most 1, from v_pk_fma_f16). LDS: row r's 16 bytes
+// of lo at 16 r, its 8 of hi at 8 r.
+template <>
+struct PfW<TF_HIP_TYPE_Q6_K> {
+    static constexpr int kBytes = 16, kBytes2 = 8, kSub = 256, kScale = 2;
+    static constexpr bool kMin = false, kPair = true;
+    struct Raw {
+        uint2 lo, hi;
+    };
+    __device__ static int off(int c) { return 8 * (c & 1); }
+    __device__ static Raw load(const TF_GLOBAL uint8_t* p, const TF_GLOBAL uint8_t* p2) {
+        return {gload_u2((const void*)p), gload_u2((const void*)p2)};
+    }
+    __device__ static Raw lds(const unsigned char* p, const unsigned char* p2, int r, int c) {
+        return {*(const uint2*)(p + 16 * r + 8 * (c & 1)), *(const uint2*)(p2 + 8 * r)};
+    }
+    // word: the scale bytes of blocks 2 p, 2 p + 1 (j: which of the two)
+    __device__ static void cvt(const Raw& w, uint32_t word, int j, int c, h8_t& bh, h8_t& bl) {
+        const int sh = 4 * (c >> 1), hs = 2 * c;
+        const uint32_t u0 = ((w.lo.x >> sh) & 0x0F0F0F0Fu) | (((w.hi.x >> hs) & 0x03030303u) << 4);
+        const uint32_t u1 = ((w.lo.y >> sh) & 0x0F0F0F0Fu) | (((w.hi.y >> hs) & 0x03030303u) << 4);
+        const tf_u32x4 p = {bytes_to_h2(u0, 0), bytes_to_h2(u0, 1), bytes_to_h2(u1, 0), bytes_to_h2(u1, 1)};
+        const h8_t off = {1056, 1056, 1056, 1056, 1056, 1056, 1056, 1056};
+        const h8_t q = __builtin_bit_cast(h8_t, p) - off;  // u - 32, exact
+        const _Float16 sc = (_Float16)(int8_t)(word >> (16 * j + 8 * (c >> 1)));
+        const h8_t scv = {sc, sc, sc, sc, sc, sc, sc, sc};
+        bh = q * scv;
+        bl = __builtin_elementwise_fma(q, scv, -bh);
+    }
 };
 
 // Block blk's scale d and min m from a scale word: a pair of fp16 d (blocks 2 p, 2 p + 1)
@@ -281,7 +323,7 @@ __global__ __launch_bounds__(kBlock) void k_pf_split(const float* x, int64_t ldx
 // Field of the segment holding output subtile u (uniform per wave: scalar selects).
 #define PF_SEL(s, f) ((s) == 0 ? a.seg[0].f : ((s) == 1 ? a.seg[1].f : a.seg[2].f))
 
-// A register-streamed tile (k_pf_gemm_tile, k_pf_gemm_f32, k_pf_gemm_q6k): a workgroup of 4
+// A register-streamed tile (k_pf_gemm_tile, k_pf_gemm_f32): a workgroup of 4
 // waves as 2 (rows) x 2 (columns); a wave owns 32 rows from m0 and NI weight-column subtiles
 // of 16 (GEMV_SILU: NI / 2 output subtiles, each a gate and an up subtile). Per subtile: its
 // segment, the weight row c this lane reads (the output column), whether it is past the
@@ -405,18 +447,27 @@ struct TileCtx {
 // same two MFMAs against a fragment of ones). Weight bytes and activation fragments stream
 // from L2 into registers, one stage of two blocks ahead; every load is unconditional
 // (indices clamped) so the compiler waits only for the stage it consumes.
+// Q6_K: a third MFMA takes the activations' hi against the weights' lo (lo x lo is below 2^-22
+// of the product), and d comes from a stream of its own, one per eight blocks. (Q6_K ran on a
+// kernel of its own with one block's loads in flight and no K slices, bound by their latency: a
+// 129-token prompt of the Llama-3.2-1B shape took 12.0 ms, 3.5 on this kernel and the large tiles.)
 template <int MODE, int NI, int T, bool SPLIT, int MI, int WM>
 __global__ __launch_bounds__(256) void k_pf_gemm_tile(const PfGemmArgs a) {
     using W = PfW<T>;
     const TileCtx<MODE, NI, MI, WM> t(a, SPLIT ? a.ks : 1);
     const int K = a.K, nblk = K / 32;
     constexpr int SW = W::kScale == 4 ? 2 : 1;  // scale words per stage and column
-    const TF_GLOBAL uint8_t* bp[NI];
+    const TF_GLOBAL uint8_t *bp[NI], *bp2[NI];
     const TF_GLOBAL uint32_t* sp[NI];
+    const TF_GLOBAL uint16_t* dp[NI];
 #pragma unroll
     for (int ni = 0; ni < NI; ++ni) {
         bp[ni] = (const TF_GLOBAL uint8_t*)t.wq[ni] + (int64_t)t.c[ni] * nblk * W::kBytes + W::off(t.lc);
         sp[ni] = (const TF_GLOBAL uint32_t*)(t.ws[ni] + (int64_t)t.c[ni] * nblk * W::kScale);
+        if constexpr (W::kPair) {
+            bp2[ni] = (const TF_GLOBAL uint8_t*)t.wq2[ni] + (int64_t)t.c[ni] * nblk * W::kBytes2;
+            dp[ni] = (const TF_GLOBAL uint16_t*)(t.ws2[ni] + (int64_t)t.c[ni] * (nblk / 8) * 2);
+        }
     }
     const TF_GLOBAL h8_t* ap[MI];
     t.act(a, ap);
@@ -431,6 +482,7 @@ __global__ __launch_bounds__(256) void k_pf_gemm_tile(const PfGemmArgs a) {
         h8_t ah[MI][2], al[MI][2];  // [row subtile][block]
         typename W::Raw bw[NI][2];  // [column subtile][block]: the lane's weight bytes
         uint32_t d[NI][SW];         // the scale words of the stage's two blocks
+        uint16_t d2[NI];            // Q6_K: d of the stage's blocks
     };
     const int S = SPLIT ? K / 64 / a.ks : K / 64;  // stages (two blocks) of this K slice
     const int sb = SPLIT ? t.kslice * S : 0;       // its first stage
@@ -445,8 +497,16 @@ __global__ __launch_bounds__(256) void k_pf_gemm_tile(const PfGemmArgs a) {
                 g.al[mi][j] = ap[mi][blk * 128 + 64];
             }
 #pragma unroll
-            for (int ni = 0; ni < NI; ++ni) g.bw[ni][j] = W::load(bp[ni] + (int64_t)blk * W::kBytes);
+            for (int ni = 0; ni < NI; ++ni) {
+                if constexpr (W::kPair)
+                    g.bw[ni][j] = W::load(bp[ni] + (int64_t)blk * W::kBytes, bp2[ni] + (int64_t)blk * W::kBytes2);
+                else
+                    g.bw[ni][j] = W::load(bp[ni] + (int64_t)blk * W::kBytes);
+            }
         }
+        if (W::kPair)
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni) g.d2[ni] = dp[ni][s >> 2];
         if (W::kScale)
 #pragma unroll
             for (int ni = 0; ni < NI; ++ni)
@@ -457,9 +517,14 @@ __global__ __launch_bounds__(256) void k_pf_gemm_tile(const PfGemmArgs a) {
     auto compute = [&](const Stage& g) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            h8_t bh[NI];
+            h8_t bh[NI], bl[NI];
 #pragma unroll
-            for (int ni = 0; ni < NI; ++ni) bh[ni] = W::cvt(g.bw[ni][j], t.lc);
+            for (int ni = 0; ni < NI; ++ni) {
+                if constexpr (W::kPair)
+                    W::cvt(g.bw[ni][j], g.d[ni][0], j, t.lc, bh[ni], bl[ni]);
+                else
+                    bh[ni] = W::cvt(g.bw[ni][j], t.lc);
+            }
             f4_t tb[MI][NI], ts[MI];
 #pragma unroll
             for (int mi = 0; mi < MI; ++mi) {
@@ -478,10 +543,19 @@ __global__ __launch_bounds__(256) void k_pf_gemm_tile(const PfGemmArgs a) {
                     tb[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_f16(g.al[mi][j], bh[ni], tb[mi][ni], 0, 0, 0);
                 if (W::kMin) ts[mi] = __builtin_amdgcn_mfma_f32_16x16x32_f16(g.al[mi][j], ones, ts[mi], 0, 0, 0);
             }
+            if constexpr (W::kPair)
+#pragma unroll
+                for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+                    for (int ni = 0; ni < NI; ++ni)
+                        tb[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_f16(g.ah[mi][j], bl[ni], tb[mi][ni], 0, 0, 0);
 #pragma unroll
             for (int ni = 0; ni < NI; ++ni) {
-                float dv, mv;
-                pf_scale<W::kScale>(g.d[ni][SW == 2 ? j : 0], j, dv, mv);
+                float dv, mv = 0.0f;
+                if (W::kPair)
+                    dv = h2f(g.d2[ni]);
+                else
+                    pf_scale<W::kScale>(g.d[ni][SW == 2 ? j : 0], j, dv, mv);
 #pragma unroll
                 for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
@@ -552,76 +626,6 @@ __global__ __launch_bounds__(256) void k_pf_gemm_f32(const PfGemmArgs a) {
     t.epilogue(a, acc);
 }
 
-// Q6_K weights (quant.cpp:101-127). A 32-element group of a row: lo[16] (element e < 16 in
-// the low nibble of byte e, e + 16 in its high nibble), hi[8] (element e's top two bits at
-// bits 2 (e / 8) of byte e % 8), an int8 scale per 16 elements and an fp16 d per 256: the
-// value d sc (u - 32) for the 6-bit code u. Lane l's 8 elements 8 c .. 8 c + 7 (c = l / 16)
-// share the scale sc of sub-block c / 2, folded into the B operand: sc (u - 32), an integer
-// of at most 4096 in magnitude, is the fp16 pair hi (its rounding, v_pk_mul_f16) + lo (the
-// exact remainder, at most 1, from v_pk_fma_f16). Per block: the activation hi and lo against
-// B hi and the activation hi against B lo (the lo x lo term is below 2^-22 of the product)
-// from zero, then acc += d * block sum.
-template <int MODE, int NI>
-__global__ __launch_bounds__(256) void k_pf_gemm_q6k(const PfGemmArgs a) {
-    const TileCtx<MODE, NI> t(a);
-    const int K = a.K, nblk = K / 32;
-    const TF_GLOBAL uint8_t *lp[NI], *hp[NI], *scp[NI];
-    const TF_GLOBAL uint16_t* dp[NI];
-#pragma unroll
-    for (int ni = 0; ni < NI; ++ni) {
-        const int64_t c = t.c[ni];
-        lp[ni] = (const TF_GLOBAL uint8_t*)t.wq[ni] + c * (K / 2) + 8 * (t.lc & 1);
-        hp[ni] = (const TF_GLOBAL uint8_t*)t.wq2[ni] + c * (K / 4);
-        scp[ni] = (const TF_GLOBAL uint8_t*)t.ws[ni] + c * (K / 16) + (t.lc >> 1);
-        dp[ni] = (const TF_GLOBAL uint16_t*)(t.ws2[ni] + c * (K / 256) * 2);
-    }
-    const TF_GLOBAL h8_t* ap[2];
-    t.act(a, ap);
-    f4_t acc[2][NI];
-#pragma unroll
-    for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = (f4_t){0.0f, 0.0f, 0.0f, 0.0f};
-    const f4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int blk = 0; blk < nblk; ++blk) {
-        h8_t ah[2], al[2];
-#pragma unroll
-        for (int mi = 0; mi < 2; ++mi) {
-            ah[mi] = ap[mi][blk * 128];
-            al[mi] = ap[mi][blk * 128 + 64];
-        }
-        h8_t bh[NI], bl[NI];
-        float dv[NI];
-#pragma unroll
-        for (int ni = 0; ni < NI; ++ni) {
-            const uint2 lo = gload_u2((const void*)(lp[ni] + 16 * blk));
-            const uint2 hi = gload_u2((const void*)(hp[ni] + 8 * blk));
-            const int sh = 4 * (t.lc >> 1), hs = 2 * t.lc;
-            const uint32_t u0 = ((lo.x >> sh) & 0x0F0F0F0Fu) | (((hi.x >> hs) & 0x03030303u) << 4);
-            const uint32_t u1 = ((lo.y >> sh) & 0x0F0F0F0Fu) | (((hi.y >> hs) & 0x03030303u) << 4);
-            const tf_u32x4 p = {bytes_to_h2(u0, 0), bytes_to_h2(u0, 1), bytes_to_h2(u1, 0), bytes_to_h2(u1, 1)};
-            const h8_t off = {1056, 1056, 1056, 1056, 1056, 1056, 1056, 1056};
-            const h8_t q = __builtin_bit_cast(h8_t, p) - off;  // u - 32, exact
-            const _Float16 sc = (_Float16)(int8_t)scp[ni][2 * blk];
-            const h8_t scv = {sc, sc, sc, sc, sc, sc, sc, sc};
-            bh[ni] = q * scv;
-            bl[ni] = __builtin_elementwise_fma(q, scv, -bh[ni]);
-            dv[ni] = h2f(dp[ni][blk >> 3]);
-        }
-#pragma unroll
-        for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-            for (int ni = 0; ni < NI; ++ni) {
-                f4_t tb = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[mi], bh[ni], zero, 0, 0, 0);
-                tb = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[mi], bh[ni], tb, 0, 0, 0);
-                tb = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[mi], bl[ni], tb, 0, 0, 0);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[mi][ni][r] = fmaf(dv[ni], tb[r], acc[mi][ni][r]);
-            }
-    }
-    t.epilogue(a, acc);
-}
-
 // Large tiles for GEMMs with enough of them to fill the CUs: a workgroup of 8 waves
 // (2 rows x 4 columns of waves) owns 128 rows x 16 weight-column subtiles (256 weight rows;
 // GEMV_SILU: 8 gate and the 8 matching up subtiles, 128 output columns). A stage (one
@@ -637,17 +641,28 @@ __global__ __launch_bounds__(256) void k_pf_gemm_q6k(const PfGemmArgs a) {
 constexpr int kBigThreads = 512;
 constexpr int kBigWaves = kBigThreads / 64;
 constexpr int kBigRows = 128;
-constexpr int kBigABytes = 16 * 1024;                           // 16 activation fragments (8 row tiles, hi and lo)
-constexpr int kBigBBytes = 16 * 1024;                           // 256 weight rows x 64 bytes at most (F16)
-constexpr int kBigStageBytes = kBigABytes + kBigBBytes + 1024;  // + a scale word per weight row
-constexpr int kBigStages = 4;                                   // LDS buffers: one in use, three loading
-constexpr size_t kBigLdsBytes = kBigStages * (size_t)kBigStageBytes;
+constexpr int kBigABytes = 16 * 1024;  // 16 activation fragments (8 row tiles, hi and lo)
+constexpr int kBigStages = 4;          // LDS buffers: one in use, three loading
+// A stage's weight bytes: 256 rows x 64 at most (F16); Q6_K's two streams, lo then hi, in 8 KiB
+constexpr int big_b_bytes(int type) { return type == TF_HIP_TYPE_Q6_K ? 8 * 1024 : 16 * 1024; }
+constexpr int kBigHiOff = 4 * 1024;
+constexpr int big_stage_bytes(int type) { return kBigABytes + big_b_bytes(type) + 1024; }  // + a scale word per weight row
+// Beside the stages, Q6_K keeps d (fp16) of the workgroup's 256 weight rows for the
+// super-blocks of 8 blocks that a slice of S blocks can touch: [super-block][row].
+constexpr size_t big_lds_bytes(int type, int S) {
+    return kBigStages * (size_t)big_stage_bytes(type) + (type == TF_HIP_TYPE_Q6_K ? ((S + 7) / 8 + 1) * (size_t)512 : 0);
+}
+constexpr int kMaxK = kBlock * 8 * kSplitGroups;  // pf_gemm_supported
+static_assert(big_lds_bytes(TF_HIP_TYPE_F16, kMaxK / 32) <= 160 * 1024 &&
+                  big_lds_bytes(TF_HIP_TYPE_Q6_K, kMaxK / 32) <= 160 * 1024,
+              "a CU's LDS");
 
 // SPLIT: the grid also splits K into a.ks slices; slice ks writes its row-scaled partial
 // sums to a.part[ks][row][output column] and k_pf_reduce applies the epilogue.
 template <int MODE, bool SPLIT, int T>
 __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a) {
     using W = PfW<T>;
+    constexpr int kBigBBytes = big_b_bytes(T), kBigStageBytes = big_stage_bytes(T);
     extern __shared__ __align__(16) unsigned char lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int b = blockIdx.x;
@@ -693,6 +708,16 @@ __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a)
     }
     constexpr int NB = W::kSub == 1024 ? 2 : 1;  // weight loads per wave and stage
     const TF_GLOBAL uint8_t* bsrc[NB];
+    const TF_GLOBAL uint8_t* bsrc2 = nullptr;  // Q6_K's hi stream: lane i, dword i % 2 of row 32 wave + i / 2
+    if constexpr (W::kPair) {
+        const int j = 32 * wave + (lane >> 1), q = j / 16;
+        int u, seg;
+        bool up;
+        resolve(q, u, seg, up);
+        const uint8_t* wq2 = up ? PF_SEL(seg, w2.q2) : PF_SEL(seg, w.q2);
+        bsrc2 = (const TF_GLOBAL uint8_t*)wq2 +
+                ((int64_t)(u - PF_SEL(seg, sub0)) * 16 + (j & 15)) * nblk * W::kBytes2 + 4 * (lane & 1);
+    }
     if (W::kSub == 512) {
         bsrc[0] = wrow(2 * wave + (lane >> 5), l16, 16 * (lc & 1));
     } else if (W::kSub == 256) {
@@ -727,6 +752,9 @@ __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a)
         } else if (W::kSub == 256) {
             const uint32_t m0 = __builtin_amdgcn_readfirstlane(bb + 512u * wave);
             if (lane < 32) lds_dma16(bsrc[0] + (int64_t)blk * W::kBytes, m0);
+            if constexpr (W::kPair)
+                lds_dma4(bsrc2 + (int64_t)blk * W::kBytes2,
+                         __builtin_amdgcn_readfirstlane(bb + kBigHiOff + 256u * wave));
         } else {
 #pragma unroll
             for (int j = 0; j < NB; ++j)
@@ -737,8 +765,22 @@ __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a)
             if (lane < 32) lds_dma4(dsrc + (W::kScale == 2 ? blk / 2 : blk), m0);
         }
     };
-    constexpr int kLoads = 2 + NB + (W::kScale ? 1 : 0);
-    static_assert(kLoads == 4, "the waits below count 4 loads per stage");
+    constexpr int kLoads = 2 + NB + (W::kScale ? 1 : 0) + (W::kPair ? 1 : 0);
+    static_assert(kLoads == (W::kPair ? 5 : 4), "the waits below count 4 (5) loads per stage");
+    // Q6_K: the d table, in LDS before the first stage's barrier
+    unsigned char* dtab = lds + kBigStages * kBigStageBytes;
+    if constexpr (W::kPair) {
+        const int sb0 = s0 / 8, nsb = (s0 + S - 1) / 8 - sb0 + 1;
+        for (int i = tid; i < 256 * nsb; i += kBigThreads) {
+            const int row = i & 255, q = row / 16;
+            int u, seg;
+            bool up;
+            resolve(q, u, seg, up);
+            const uint8_t* ws2 = up ? PF_SEL(seg, w2.s2) : PF_SEL(seg, w.s2);
+            const int c = (u - PF_SEL(seg, sub0)) * 16 + (row & 15);
+            ((uint16_t*)dtab)[i] = ((const TF_GLOBAL uint16_t*)ws2)[(int64_t)c * (nblk / 8) + sb0 + (i >> 8)];
+        }
+    }
 
     const int wm = wave & 1, wn = wave >> 1;
     int qb[4];  // this wave's weight-column subtiles
@@ -776,11 +818,18 @@ __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a)
         const unsigned char* sb = lds + buf * kBigStageBytes + kBigABytes;
         const uint32_t* sd = (const uint32_t*)(lds + buf * kBigStageBytes + kBigABytes + kBigBBytes);
         float dv[4], mv[4];
-        h8_t bh[4];
+        h8_t bh[4], bl[4];
 #pragma unroll
         for (int ni = 0; ni < 4; ++ni) {
-            pf_scale<W::kScale>(W::kScale ? sd[qb[ni] * 16 + l16] : 0u, blk, dv[ni], mv[ni]);
-            bh[ni] = W::cvt(W::lds(sb + qb[ni] * W::kSub, l16, lc), lc);
+            if constexpr (W::kPair) {
+                dv[ni] = h2f(((const uint16_t*)dtab)[(blk / 8 - s0 / 8) * 256 + qb[ni] * 16 + l16]);
+                mv[ni] = 0.0f;
+                W::cvt(W::lds(sb + qb[ni] * W::kSub, sb + kBigHiOff + qb[ni] * 128, l16, lc), sd[qb[ni] * 16 + l16],
+                       blk & 1, lc, bh[ni], bl[ni]);
+            } else {
+                pf_scale<W::kScale>(W::kScale ? sd[qb[ni] * 16 + l16] : 0u, blk, dv[ni], mv[ni]);
+                bh[ni] = W::cvt(W::lds(sb + qb[ni] * W::kSub, l16, lc), lc);
+            }
         }
         auto mfmas = [&](int half, f4_t (&t)[2][4], f4_t (&ts)[2]) {
             h8_t ah[2], al[2];
@@ -806,6 +855,12 @@ __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a)
                     t[mm][ni] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[mm], bh[ni], t[mm][ni], 0, 0, 0);
                 if (W::kMin) ts[mm] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[mm], ones, ts[mm], 0, 0, 0);
             }
+            if constexpr (W::kPair)
+#pragma unroll
+                for (int mm = 0; mm < 2; ++mm)
+#pragma unroll
+                    for (int ni = 0; ni < 4; ++ni)
+                        t[mm][ni] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[mm], bl[ni], t[mm][ni], 0, 0, 0);
         };
         f4_t t0[2][4], ts0[2];
         mfmas(0, t0, ts0);
@@ -827,9 +882,9 @@ __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a)
         // wave has left compute(s - 1), whose buffer stage s + 3 takes
         const int after = S - 1 - s;
         if (after >= 2)
-            asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * kLoads) : "memory");
         else if (after == 1)
-            asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kLoads) : "memory");
         else
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
         if (s + kBigStages - 1 < S) issue(s + kBigStages - 1);
@@ -1756,21 +1811,22 @@ hipError_t launch_gemm_t(const PfGemmArgs& a, hipStream_t st, bool* fused) {
                                   (const void*)k_pf_gemm_big<GEMV_SILU, true, T>};
             const int fi = a.mode + (ks > 1 ? 3 : 0);
             if (!attr_set[fi]) {
-                const hipError_t e =
-                    hipFuncSetAttribute(fns[fi], hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBigLdsBytes);
+                const hipError_t e = hipFuncSetAttribute(fns[fi], hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                         (int)big_lds_bytes(T, kMaxK / 32));
                 if (e != hipSuccess) return e;
                 attr_set[fi] = true;
             }
             PfGemmArgs b = a;
             b.ks = ks;
             const dim3 grid((unsigned)(n_big * ks));
+            const size_t lds = big_lds_bytes(T, a.K / 32 / ks);
             switch (fi) {
-                case 0: hipLaunchKernelGGL((k_pf_gemm_big<GEMV_STORE, false, T>), grid, dim3(kBigThreads), kBigLdsBytes, st, b); break;
-                case 1: hipLaunchKernelGGL((k_pf_gemm_big<GEMV_RESID, false, T>), grid, dim3(kBigThreads), kBigLdsBytes, st, b); break;
-                case 2: hipLaunchKernelGGL((k_pf_gemm_big<GEMV_SILU, false, T>), grid, dim3(kBigThreads), kBigLdsBytes, st, b); break;
-                case 3: hipLaunchKernelGGL((k_pf_gemm_big<GEMV_STORE, true, T>), grid, dim3(kBigThreads), kBigLdsBytes, st, b); break;
-                case 4: hipLaunchKernelGGL((k_pf_gemm_big<GEMV_RESID, true, T>), grid, dim3(kBigThreads), kBigLdsBytes, st, b); break;
-                default: hipLaunchKernelGGL((k_pf_gemm_big<GEMV_SILU, true, T>), grid, dim3(kBigThreads), kBigLdsBytes, st, b); break;
+                case 0: hipLaunchKernelGGL((k_pf_gemm_big<GEMV_STORE, false, T>), grid, dim3(kBigThreads), lds, st, b); break;
+                case 1: hipLaunchKernelGGL((k_pf_gemm_big<GEMV_RESID, false, T>), grid, dim3(kBigThreads), lds, st, b); break;
+                case 2: hipLaunchKernelGGL((k_pf_gemm_big<GEMV_SILU, false, T>), grid, dim3(kBigThreads), lds, st, b); break;
+                case 3: hipLaunchKernelGGL((k_pf_gemm_big<GEMV_STORE, true, T>), grid, dim3(kBigThreads), lds, st, b); break;
+                case 4: hipLaunchKernelGGL((k_pf_gemm_big<GEMV_RESID, true, T>), grid, dim3(kBigThreads), lds, st, b); break;
+                default: hipLaunchKernelGGL((k_pf_gemm_big<GEMV_SILU, true, T>), grid, dim3(kBigThreads), lds, st, b); break;
             }
             hipError_t e = hipGetLastError();
             if (e != hipSuccess || ks == 1) return e;
@@ -1780,14 +1836,14 @@ hipError_t launch_gemm_t(const PfGemmArgs& a, hipStream_t st, bool* fused) {
     // 64-row tiles with two waves along the rows, or, for at most 32 rows, tiles of 16 rows
     // (at most 16) or 32 with all four waves along the columns (fewer activation reads per
     // weight byte); 4 column subtiles per wave, 2 when that leaves fewer than two workgroups
-    // per CU
+    // per CU (and for Q6_K: 4 subtiles of fp16 pairs take a SIMD's whole register file)
     const int cus = device_cu_count();
     const int shape = a.M <= 16 ? 1 : (a.M <= kSmallRows ? 2 : 0);  // 16-row, 32-row or 64-row tiles
     const int mt = shape == 0 ? a.Mpad / kPfTileM : (a.M + 16 * shape - 1) / (16 * shape);
     const int wcols = shape ? 4 : 2;  // waves along the columns
     const int out4 = a.mode == GEMV_SILU ? 2 : 4;
     const int wg4 = (a.n_sub + wcols * out4 - 1) / (wcols * out4) * mt;
-    const int ni = wg4 >= 2 * cus ? 4 : 2;
+    const int ni = wg4 >= 2 * cus && !PfW<T>::kPair ? 4 : 2;
     const int per_wg = wcols * (a.mode == GEMV_SILU ? ni / 2 : ni);  // output subtiles per workgroup column
     const int n_wg = (a.n_sub + per_wg - 1) / per_wg * mt;
     // Few tiles (a short prompt: every weight byte is read once whatever the row count, so
@@ -1858,7 +1914,7 @@ hipError_t launch_pf_gemm(const PfGemmArgs& a, hipStream_t st, bool* fused) {
         if (a.mode == GEMV_SILU && (g.w2.type != t || g.w2.K != a.K || g.w2.N != g.w.N)) return hipErrorInvalidValue;
     }
     if (a.seg[0].sub0 != 0 || (a.mode == GEMV_SILU && a.n_seg != 1)) return hipErrorInvalidValue;
-    if (t == TF_HIP_TYPE_F32 || t == TF_HIP_TYPE_Q6_K) {
+    if (t == TF_HIP_TYPE_F32) {
         // register-streamed tiles only: 4 column subtiles per wave, 2 when that leaves
         // fewer than two workgroups per CU
         const int mt = a.Mpad / kPfTileM;
@@ -1867,24 +1923,17 @@ hipError_t launch_pf_gemm(const PfGemmArgs& a, hipStream_t st, bool* fused) {
         const int ni = wg4 >= 2 * device_cu_count() ? 4 : 2;
         const int per_wg = 2 * (a.mode == GEMV_SILU ? ni / 2 : ni);
         const dim3 grid((unsigned)((a.n_sub + per_wg - 1) / per_wg * mt));
-#define PF_OWN(KERNEL, MODE, NI) hipLaunchKernelGGL((KERNEL<MODE, NI>), grid, dim3(256), 0, st, a)
-#define PF_OWN_ALL(KERNEL)                                             \
-    switch (a.mode * 8 + ni) {                                         \
-        case GEMV_STORE * 8 + 4: PF_OWN(KERNEL, GEMV_STORE, 4); break; \
-        case GEMV_STORE * 8 + 2: PF_OWN(KERNEL, GEMV_STORE, 2); break; \
-        case GEMV_RESID * 8 + 4: PF_OWN(KERNEL, GEMV_RESID, 4); break; \
-        case GEMV_RESID * 8 + 2: PF_OWN(KERNEL, GEMV_RESID, 2); break; \
-        case GEMV_SILU * 8 + 4: PF_OWN(KERNEL, GEMV_SILU, 4); break;   \
-        case GEMV_SILU * 8 + 2: PF_OWN(KERNEL, GEMV_SILU, 2); break;   \
-        default: return hipErrorInvalidValue;                          \
-    }
-        if (t == TF_HIP_TYPE_F32) {
-            PF_OWN_ALL(k_pf_gemm_f32)
-        } else {
-            PF_OWN_ALL(k_pf_gemm_q6k)
+#define PF_F32(MODE, NI) hipLaunchKernelGGL((k_pf_gemm_f32<MODE, NI>), grid, dim3(256), 0, st, a)
+        switch (a.mode * 8 + ni) {
+            case GEMV_STORE * 8 + 4: PF_F32(GEMV_STORE, 4); break;
+            case GEMV_STORE * 8 + 2: PF_F32(GEMV_STORE, 2); break;
+            case GEMV_RESID * 8 + 4: PF_F32(GEMV_RESID, 4); break;
+            case GEMV_RESID * 8 + 2: PF_F32(GEMV_RESID, 2); break;
+            case GEMV_SILU * 8 + 4: PF_F32(GEMV_SILU, 4); break;
+            case GEMV_SILU * 8 + 2: PF_F32(GEMV_SILU, 2); break;
+            default: return hipErrorInvalidValue;
         }
-#undef PF_OWN_ALL
-#undef PF_OWN
+#undef PF_F32
         return hipGetLastError();
     }
     switch (t) {
@@ -1892,6 +1941,7 @@ hipError_t launch_pf_gemm(const PfGemmArgs& a, hipStream_t st, bool* fused) {
         case TF_HIP_TYPE_Q4_0: return launch_gemm_t<TF_HIP_TYPE_Q4_0>(a, st, fused);
         case TF_HIP_TYPE_Q4_1: return launch_gemm_t<TF_HIP_TYPE_Q4_1>(a, st, fused);
         case TF_HIP_TYPE_F16: return launch_gemm_t<TF_HIP_TYPE_F16>(a, st, fused);
+        case TF_HIP_TYPE_Q6_K: return launch_gemm_t<TF_HIP_TYPE_Q6_K>(a, st, fused);
     }
     return hipErrorInvalidValue;
 }

@@ -124,11 +124,14 @@ PF_GEMM_SHAPES = [(2, 64, 16), (37, 2048, 256), (64, 896, 1152), (100, 8192, 128
 
 # the other formats the matrix cores take, read in their own layout: the register-streamed
 # tiles, the LDS-staged tiles (500 x 256 x 16384) and K split in slices (512 x 2048 x 2048);
-# F32 (0) and Q6_K (14, rows of a multiple of 256) always on their register-streamed tiles
+# F32 (0) always on its register-streamed tiles; Q6_K (14, rows of a multiple of 256) also with an
+# odd number of 256-element super-blocks a row, K slices that start inside one (1280 in 4 or 16),
+# and column tiles that the last workgroup only fills in part
 PF_GEMM_FMT_SHAPES = [(t, m, k, n) for t in (2, 3, 1, 0, 14)
                       for (m, k, n) in [(2, 64, 16), (37, 2048, 256), (130, 1536, 48), (7, 192, 320),
                                         (500, 256, 16384), (512, 2048, 2048)]
-                      if t != 14 or k % 256 == 0]
+                      if t != 14 or k % 256 == 0] + [
+    (14, m, k, n) for (m, k, n) in [(16, 1280, 48), (17, 768, 144), (128, 1280, 2064), (300, 768, 8208), (129, 2304, 272)]]
 
 
 @pytest.mark.parametrize("t,m,k,n", [(8, m, k, n) for (m, k, n) in PF_GEMM_SHAPES] + PF_GEMM_FMT_SHAPES)
