@@ -95,6 +95,8 @@ struct tf_hip_ctx {
     uint16_t* pxa = nullptr;            // activation fragments (hi, lo) of one chunk
     float* ppart = nullptr;             // split-K partial sums of the prefill GEMMs
     size_t ppart_floats = 0;
+    bool pf_small = false;              // prompts of at most kPfSmallRows take prefill_small
+    int* pf_count = nullptr;            // prefill_small's counts of finished K slices, zero between launches
     void* pattn_ws = nullptr;           // packed key/value tiles of prefill attention
     size_t pattn_ws_bytes = 0;
     std::string err;
@@ -632,13 +634,16 @@ int ensure_pf(tf_hip_ctx* c) {
     int rc = check_ready(c);
     if (rc) return rc;
     c->pf_state = 0;
+    c->pf_small = true;
     const tf_hip_hparams& p = c->hp;
     for (int l = 0; l < p.n_layer; ++l) {
         auto M = [&](int k) -> const DevMat& { return mat(c, TF_HIP_SLOT_LAYER(l, k)); };
         const int kinds[7] = {TF_HIP_LAYER_Q,    TF_HIP_LAYER_K,  TF_HIP_LAYER_V,   TF_HIP_LAYER_O,
                               TF_HIP_LAYER_GATE, TF_HIP_LAYER_UP, TF_HIP_LAYER_DOWN};
-        for (int k : kinds)
+        for (int k : kinds) {
             if (!pf_gemm_supported(M(k).type, M(k).K, M(k).N)) return 0;
+            if (M(k).type == TF_HIP_TYPE_F32) c->pf_small = false;
+        }
         // gate and up run in one launch, which takes one format
         if (M(TF_HIP_LAYER_GATE).type != M(TF_HIP_LAYER_UP).type) return 0;
     }
@@ -655,6 +660,9 @@ int ensure_pf(tf_hip_ctx* c) {
         // up to 8 K slices of the widest non-SILU output (QKV or d_model)
         c->ppart_floats = 8 * (size_t)cap * std::max(NQ, D);
         if ((rc = dalloc(c, &c->ppart, c->ppart_floats * 4))) return rc;
+        const size_t count_bytes = D / 16 * sizeof(int);
+        if ((rc = dalloc(c, &c->pf_count, count_bytes))) return rc;
+        HIPCHK(c, hipMemset(c->pf_count, 0, count_bytes));
         // attention of a chunk covers at most max_seq positions
         c->pattn_ws_bytes = pf_attn_ws_bytes(p.head_dim, p.n_kv_head, p.max_seq);
         if ((rc = dalloc(c, &c->pattn_ws, c->pattn_ws_bytes))) return rc;
@@ -684,6 +692,92 @@ DevMat devmat_rows(const DevMat& m, int64_t r0, int64_t n) {
     d.s2 = m.s2 ? m.s2 + r0 * s2 : nullptr;
     d.N = n;
     return d;
+}
+
+// n <= kPfSmallRows prompt tokens, staged at hist[c->pos ..], through the layers, ending with
+// the lm_head of the last row, as prefill_mfma.
+int prefill_small(tf_hip_ctx* c, int n) {
+    const tf_hip_hparams& p = c->hp;
+    const int D = p.n_embd, F = p.n_ff, Hd = c->H, KVd = c->KVd, NQ = Hd + 2 * KVd;
+    // the residual rows' operand, then that of the attention output or the hidden rows; their
+    // sums of squares where longer prompts keep K slices (ensure_pf sized both for 128 rows)
+    uint16_t* xa = c->pxa;
+    uint16_t* ha = c->pxa + kPfSmallOperand((size_t)D);
+    double* ssp = (double*)c->ppart;
+    float* part = c->ppart + 2 * kPfSmallRows * (size_t)(D / 16);
+    hipError_t e = launch_embed_rows(mat(c, TF_HIP_SLOT_TOKEN_EMBD), c->hist + c->pos, n, c->px, D, c->st);
+    auto chk = [&](hipError_t r) {
+        if (e == hipSuccess) e = r;
+    };
+    auto base = [&](const uint16_t* in, int K, int mode) {
+        PfSmallArgs a;
+        a.xa = in;
+        a.ssp = mode == GEMV_RESID ? nullptr : ssp;
+        a.K = K;
+        a.M = n;
+        a.mode = mode;
+        a.eps = p.rms_eps;
+        return a;
+    };
+    auto seg = [&](PfSmallArgs& a, const DevMat& w, float* y, int64_t ldy, const float* bias) {
+        PfSeg& s = a.seg[a.n_seg++];
+        s.w = w;
+        s.y = y;
+        s.ldy = ldy;
+        s.bias = bias;
+        s.sub0 = a.n_sub;
+        a.n_sub += (int)(w.N / 16);
+    };
+    // the updated residual rows as the operand behind the rmsnorm with norm_w
+    auto next = [&](PfSmallArgs& a, const float* norm_w) {
+        a.oxa = xa;
+        a.onorm_w = norm_w;
+        a.ossp = ssp;
+    };
+    auto slices = [&](PfSmallArgs& a) {
+        a.part = part;
+        a.count = c->pf_count;
+    };
+    chk(launch_pf_small_split(c->px, D, n, vec(c, TF_HIP_SLOT_LAYER(0, TF_HIP_LAYER_ATTN_NORM)), xa, ssp, c->st));
+    for (int l = 0; l < p.n_layer && e == hipSuccess; ++l) {
+        auto M = [&](int k) -> const DevMat& { return mat(c, TF_HIP_SLOT_LAYER(l, k)); };
+        auto V = [&](int k) { return vec(c, TF_HIP_SLOT_LAYER(l, k)); };
+        // q, k and v: a launch per run of matrices in one format
+        const int kinds[3] = {TF_HIP_LAYER_Q, TF_HIP_LAYER_K, TF_HIP_LAYER_V};
+        const int bias[3] = {TF_HIP_LAYER_BQ, TF_HIP_LAYER_BK, TF_HIP_LAYER_BV};
+        const int off[3] = {0, Hd, Hd + KVd};
+        for (int i = 0; i < 3;) {
+            PfSmallArgs a = base(xa, D, GEMV_STORE);
+            const int t = M(kinds[i]).type;
+            for (; i < 3 && M(kinds[i]).type == t; ++i) seg(a, M(kinds[i]), c->pqkv + off[i], NQ, V(bias[i]));
+            chk(launch_pf_small(a, c->st));
+        }
+        const PfSmallAttn at{c->pqkv, NQ, c->rope_cos, c->rope_sin, c->kc + (size_t)l * c->kv_layer,
+                             c->vc + (size_t)l * c->kv_layer, ha, n, c->pos, p.n_head, p.n_kv_head, p.kv_layout,
+                             p.max_seq};
+        chk(launch_pf_small_attn(at, p.head_dim, c->st));
+        PfSmallArgs o = base(ha, Hd, GEMV_RESID);
+        seg(o, M(TF_HIP_LAYER_O), c->px, D, nullptr);
+        next(o, V(TF_HIP_LAYER_FFN_NORM));
+        slices(o);
+        chk(launch_pf_small(o, c->st));
+        PfSmallArgs gu = base(xa, D, GEMV_SILU);
+        seg(gu, M(TF_HIP_LAYER_GATE), nullptr, 0, nullptr);
+        gu.seg[0].w2 = M(TF_HIP_LAYER_UP);
+        gu.oxa = ha;
+        chk(launch_pf_small(gu, c->st));
+        PfSmallArgs dn = base(ha, F, GEMV_RESID);
+        seg(dn, M(TF_HIP_LAYER_DOWN), c->px, D, nullptr);
+        dn.tap = c->taps + (size_t)l * D;
+        dn.tap_row = n - 1;
+        slices(dn);
+        if (l + 1 < p.n_layer) next(dn, vec(c, TF_HIP_SLOT_LAYER(l + 1, TF_HIP_LAYER_ATTN_NORM)));
+        chk(launch_pf_small(dn, c->st));
+    }
+    chk(launch_pf_tail(c->ctl, c->pos + n - 1, c->hist, c->px + (size_t)(n - 1) * D, c->x, D, c->st));
+    chk(launch_lm_head(c));
+    if (e != hipSuccess) return fail(c, TF_HIP_EDEVICE, std::string("prefill launch: ") + hipGetErrorString(e));
+    return 0;
 }
 
 // n prompt tokens, staged at hist[c->pos ..], through the matrix-core layers in chunks
@@ -1118,7 +1212,7 @@ int tf_hip_prefill(tf_hip_ctx* c, const int32_t* tokens, int32_t n, float* logit
     if ((rc = set_ctl(c, c->pos, 0))) return rc;
     HIPCHK(c, hipEventRecord(c->ev0, c->st));
     if (use_pf) {
-        if ((rc = prefill_mfma(c, n))) return rc;
+        if ((rc = n <= kPfSmallRows && c->pf_small ? prefill_small(c, n) : prefill_mfma(c, n))) return rc;
     } else if ((rc = run_tokens(c, &use_step, n, 0, 0, c->pos))) {
         return rc;
     }

@@ -206,6 +206,48 @@ struct PfGemmArgs {
     int pos0 = 0, n_head = 0, n_kv = 0, hd = 0, kv_layout = 0, max_seq = 0;
 };
 
+// Prompts of at most kPfSmallRows rows (k_pf_small.hip). The GEMMs' operands are bf16 triples in
+// fragment order, kPfSmallOperand(K) halves for rows of K; a GEMM writes the next one's operand
+// (oxa; times onorm_w where an rmsnorm stands between them, with its sums of squares in ossp).
+constexpr int kPfSmallRows = 16;  // one MFMA row tile
+constexpr size_t kPfSmallOperand(size_t K) { return 3 * kPfSmallRows * K; }
+struct PfSmallArgs {
+    const uint16_t* xa = nullptr;
+    const double* ssp = nullptr;  // sums of squares [K / 16][kPfSmallRows], not for GEMV_RESID
+    float eps = 0.0f;
+    int K = 0, M = 0;
+    PfSeg seg[3];                 // y is not used by GEMV_SILU
+    int n_seg = 0, n_sub = 0;     // 16-column output tiles over all segments
+    int mode = GEMV_STORE;        // GEMV_STORE, GEMV_RESID or GEMV_SILU
+    float* tap = nullptr;         // GEMV_RESID: copy of output row tap_row
+    int tap_row = -1;
+    uint16_t* oxa = nullptr;
+    const float* onorm_w = nullptr;
+    double* ossp = nullptr;
+    // GEMV_RESID may take K in up to kPfSmallSlices slices: their sums (kPfSmallPart floats) and a
+    // count per tile group (zero before and after every launch), or nullptr
+    float* part = nullptr;
+    int* count = nullptr;
+    int ks = 1;  // set by launch_pf_small
+};
+constexpr int kPfSmallSlices = 8;
+constexpr size_t kPfSmallPart(size_t N) { return kPfSmallSlices * kPfSmallRows * N; }
+hipError_t launch_pf_small(const PfSmallArgs& a, hipStream_t st);
+// The operand of x rows [M][D] times norm_w, and their sums of squares.
+hipError_t launch_pf_small_split(const float* x, int D, int M, const float* norm_w, uint16_t* xa, double* ssp,
+                                 hipStream_t st);
+// Attention of a prompt's n rows over themselves: raw q, k, v rows [n][ld] at position pos0;
+// the output as an operand.
+struct PfSmallAttn {
+    const float* qkv;
+    int64_t ld;
+    const float *rope_cos, *rope_sin;
+    float *kc, *vc;
+    uint16_t* oxa;
+    int n, pos0, H, G, layout, max_seq;
+};
+hipError_t launch_pf_small_attn(const PfSmallAttn& a, int hd, hipStream_t st);
+
 // Q8_0, Q4_0, Q4_1, F16, F32 or Q6_K (K % 256 == 0) with K % 64 == 0 and N % 16 == 0; the
 // matrices of one launch_pf_gemm share one format.
 bool pf_gemm_supported(int type, int64_t K, int64_t N);

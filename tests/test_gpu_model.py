@@ -246,6 +246,126 @@ def test_prefill_prompt_lengths(pkg, gguf, n_prompt):
     print(f"small_q8 {n_prompt}-token prompt: ids {ids} logits {worst:.2e} taps {worst_tap:.2e}")
 
 
+# head counts, d_model, ffn, layer formats (q, k, v, o, gate / up, down): row lengths that end in half
+# a 128-element stage (192, 320, 4160), an odd number of 16-column tiles, head sizes 32 / 64 / 128, q, k
+# and v in one to three formats, Q6_K's super-blocks, and ffn_down in K slices (8192 and 4160 long)
+SHORT_PROMPT_MODELS = [
+    (6, 2, 192, 320, (8, 8, 8, 8, 8, 8)),
+    (4, 2, 256, 8192, (2, 2, 2, 3, 2, 2)),
+    (2, 1, 256, 4160, (1, 8, 8, 1, 1, 1)),
+    (4, 4, 256, 2048, (14, 3, 2, 14, 14, 14)),
+    (8, 1, 256, 8192, (14, 14, 14, 8, 3, 3)),
+]
+
+
+@pytest.mark.parametrize("shape", SHORT_PROMPT_MODELS)
+def test_short_prompt_kernels(pkg, shape):
+    """Prompts of 2 to 16 tokens (their own kernels) and of 17: logits, taps and K/V rows no further
+    from the model in float64 than twice what the per-token prefill of the same context is, or
+    4e-6 where that is closer still (random blocks cancel, so fp32 sums in any order lose
+    digits: up to 2e-5 here); the second run of a prompt bit for bit the first (nothing is left
+    behind in the counts of the K slices)."""
+    import ctypes as C
+
+    from gpu_util import oracle_dequant
+    from rows import random_rows
+
+    heads, kv, d, ff, fmts = shape
+    hd, vocab, layers, max_seq = d // heads, 96, 2, 48
+    L, rng = pkg.hip_lib(), np.random.default_rng(d + ff)
+    hp = pkg.HParams(vocab, d, ff, layers, heads, kv, hd, max_seq, 1, 1e-5)
+    ctx = C.c_void_p()
+    assert L.tf_hip_create(0, C.cast(C.byref(hp), C.c_void_p), C.byref(ctx)) == 0
+
+    w = {}  # slot -> float64
+
+    def up(slot, t, k, n):
+        raw = random_rows(rng, t, k, n)
+        w[slot] = oracle_dequant(t, raw, k).astype(np.float64)
+        assert L.tf_hip_upload_tensor(ctx, slot, t, k, n, raw.ctypes.data, raw.nbytes) == 0
+
+    def vec(slot, n, mean):
+        v = (mean + 0.2 * rng.standard_normal(n)).astype(np.float32)
+        w[slot] = v.astype(np.float64)
+        assert L.tf_hip_upload_tensor(ctx, slot, 0, n, 1, v.ctypes.data, v.nbytes) == 0
+
+    up(0, 8, d, vocab)
+    vec(1, d, 1.0)
+    for l in range(layers):
+        s = 16 + 12 * l
+        for slot, t, k, n in ((1, fmts[0], d, d), (2, fmts[1], d, kv * hd), (3, fmts[2], d, kv * hd),
+                              (4, fmts[3], d, d), (9, fmts[4], d, ff), (10, fmts[4], d, ff), (11, fmts[5], ff, d)):
+            up(s + slot, t, k, n)
+        for slot, n, mean in ((0, d, 1.0), (8, d, 1.0), (5, d, 0.0), (6, kv * hd, 0.0)):
+            vec(s + slot, n, mean)
+    F = lambda a: a.ctypes.data_as(C.POINTER(C.c_float))  # noqa: E731
+    cos, sin = pkg.rope_tables(10000.0, hd, max_seq)
+    assert L.tf_hip_set_rope_table(ctx, F(cos), F(sin), max_seq, hd // 2) == 0
+
+    def prefill(path, tokens):
+        assert L.tf_hip_set_prefill_path(ctx, path) == 0
+        assert L.tf_hip_reset(ctx) == 0
+        n, out = len(tokens), [np.zeros(vocab, np.float32)]
+        # a first call of two tokens, so that the prompt starts past position 0
+        head = np.array([1, 2], np.int32)
+        I = C.POINTER(C.c_int32)  # noqa: E741
+        assert L.tf_hip_prefill(ctx, head.ctypes.data_as(I), 2, None, None) == 0
+        assert L.tf_hip_prefill(ctx, tokens.ctypes.data_as(I), n, F(out[0]), None) == 0
+        for l in range(layers):
+            out.append(np.zeros(d, np.float32))
+            assert L.tf_hip_get_layer_act(ctx, l, F(out[-1])) == 0
+            for which in (0, 1):
+                out.append(np.zeros((n + 2, kv, hd), np.float32))
+                assert L.tf_hip_read_kv(ctx, l, which, 0, n + 2, F(out[-1])) == 0
+        return out
+
+    def exact(tokens):
+        """prefill's outputs in float64."""
+        kvs = [[[], []] for _ in range(layers)]
+        pos = 0
+        for part in ([1, 2], tokens):
+            x, taps = w[0][np.asarray(part)], []
+            m = len(x)
+            c, s = (np.float64(t[pos:pos + m])[:, None] for t in (cos, sin))
+            rope = lambda y: np.concatenate((y[..., :hd // 2] * c - y[..., hd // 2:] * s,  # noqa: E731
+                                             y[..., :hd // 2] * s + y[..., hd // 2:] * c), -1)
+            norm = lambda y, g: y / np.sqrt((y * y).mean(-1, keepdims=True) + np.float32(1e-5)) * g  # noqa: E731
+            for l in range(layers):
+                W = lambda k: w[16 + 12 * l + k]  # noqa: E731
+                y = norm(x, W(0))
+                q = rope((y @ W(1).T + W(5)).reshape(m, heads, hd))
+                k, v = rope((y @ W(2).T + W(6)).reshape(m, kv, hd)), (y @ W(3).T).reshape(m, kv, hd)
+                kvs[l][0].append(k)
+                kvs[l][1].append(v)
+                a = np.zeros((m, heads, hd))
+                for h in range(heads):
+                    sc = q[:, h] @ k[:, h * kv // heads].T / np.sqrt(hd)
+                    sc[np.triu_indices(m, 1)] = -np.inf
+                    e = np.exp(sc - sc.max(1, keepdims=True))
+                    a[:, h] = e / e.sum(1, keepdims=True) @ v[:, h * kv // heads]
+                x = x + a.reshape(m, d) @ W(4).T
+                y = norm(x, W(8))
+                g = y @ W(9).T
+                x = x + (g / (1 + np.exp(-g)) * (y @ W(10).T)) @ W(11).T
+                taps.append(x[-1])
+            pos += m
+        out = [w[0] @ norm(x[-1], w[1])]
+        for l in range(layers):
+            out += [taps[l]] + [np.concatenate(r) for r in kvs[l]]
+        return out
+
+    try:
+        assert L.tf_hip_get_prefill_path(ctx) == MFMA
+        for n in (2, 3, 4, 5, 8, 9, 15, 16, 17):
+            tokens = rng.integers(0, vocab, n).astype(np.int32)
+            want, got, again = prefill(TOKENS, tokens), prefill(MFMA, tokens), prefill(MFMA, tokens)
+            for i, (e, a, b, c) in enumerate(zip(exact(tokens), want, got, again)):
+                assert rel_err(b, e) <= max(2 * rel_err(a, e), 4e-6), (n, i, rel_err(b, e), rel_err(a, e))
+                assert np.array_equal(b.view(np.uint32), c.view(np.uint32)), (n, i)
+    finally:
+        L.tf_hip_destroy(ctx)
+
+
 @pytest.mark.parametrize("n_prompt", [6, 150])
 @pytest.mark.parametrize("preset", ["tiny_mixq4", "tiny_mixfmt"])
 def test_mixed_format_prefill(pkg, gguf, preset, n_prompt):
