@@ -1012,7 +1012,7 @@ __global__ __launch_bounds__(kT, 1) void k_step(const StepArgs args) {
                 // waves give 5 or 4 instead of 3 or 2 pairs, and two streams per wave keep
                 // enough loads in flight), two for the 4-bit formats (their rows are half the
                 // bytes; one row per group measured 1.8% slower on the mixed-Q4 model)
-                constexpr int kGuR = TL == TF_HIP_TYPE_Q8_0 ? 1 : 2;
+                constexpr int kGuR = TL == TF_HIP_TYPE_Q8_0 || TL == TF_HIP_TYPE_F16 ? 1 : 2;
                 const int gu_groups[3] = {(int)((ly.wg.N + kGuR - 1) / kGuR), 0, 0};
                 auto gu_seg = [&](int, int what) -> const DevMat& { return what == 1 ? ly.wu : ly.wg; };
                 auto gu_epi = [&](int, int row, float v, float up, float) {

@@ -297,6 +297,9 @@ int step_alt_type(int tl);
 hipError_t launch_step(const StepArgs& a, int type_layers, int type_out, int n_wg, hipStream_t st);
 // the Q8_0 builds with ffn_down split over K (stage_lds 2)
 hipError_t launch_step_split(const StepArgs& a, int n_wg, hipStream_t st);
+// the F16 and Q6_K builds
+hipError_t launch_step_f16(const StepArgs& a, int n_wg, hipStream_t st);
+hipError_t launch_step_q6k(const StepArgs& a, int n_wg, hipStream_t st);
 
 // Launchers (k_*.hip).
 hipError_t launch_gemv(const GemvArgs& a, int rows_per_wave, hipStream_t st);

@@ -112,7 +112,7 @@ int tf_hip_generate(tf_hip_ctx* ctx, int32_t n, int32_t* out_tokens);
 
 /* Decode path of prefill / decode / generate. TF_HIP_PATH_STEP (the default): one
  * persistent cooperative kernel per call runs every token of the call, for models whose
- * layer matrices share one format the kernel is compiled for (Q8_0, F32, or Q4_0 with
+ * layer matrices share one format the kernel is compiled for (Q8_0, F16, Q6_K, F32, or Q4_0 with
  * Q4_1 wo / ffn_down allowed; others use the graph path; tokens attending more than
  * split_from positions, 64 by default, split each layer's attention over workgroups,
  * shorter spans run it on one workgroup per kv head; see tf_hip_set_split_from).

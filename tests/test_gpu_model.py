@@ -366,6 +366,65 @@ def test_short_prompt_kernels(pkg, shape):
         L.tf_hip_destroy(ctx)
 
 
+# type, query heads, kv heads, d_model, ffn, max_seq, prompt: rows shorter and longer than a tile, rows
+# that do not fill one (192, 320), head sizes 32, 64 and 128, odd ffn row counts for the row groups,
+# attention on one workgroup per kv head and split over workgroups
+STEP_FORMATS = [
+    (1, 6, 2, 192, 320, 64, 5), (1, 2, 1, 256, 1056, 1024, 70), (1, 8, 2, 512, 4160, 64, 5), (1, 8, 8, 1024, 64, 600, 90),
+    (14, 4, 2, 256, 512, 64, 5), (14, 2, 1, 256, 768, 1024, 70), (14, 8, 1, 256, 8192, 64, 5), (14, 16, 4, 1280, 256, 600, 90),
+]
+
+
+@pytest.mark.parametrize("shape", STEP_FORMATS)
+def test_step_kernel_f16_and_q6k(pkg, shape):
+    """F16 and Q6_K models decode on the persistent step kernel: 12 greedy tokens as the graph
+    path's, logits and K/V rows of the last within 1e-5 of its (the same products summed in another
+    order: 4 sqrt(8192) eps, times two layers)."""
+    import ctypes as C
+
+    t, heads, kv, d, ff, max_seq, n_prompt = shape
+    hd, vocab, layers = d // heads, 96, 2
+    L, rng = pkg.hip_lib(), np.random.default_rng(d + ff + t)
+    hp = pkg.HParams(vocab, d, ff, layers, heads, kv, hd, max_seq, 0, 1e-5)
+    ctx = C.c_void_p()
+    assert L.tf_hip_create(0, C.cast(C.byref(hp), C.c_void_p), C.byref(ctx)) == 0
+    F = lambda a: a.ctypes.data_as(C.POINTER(C.c_float))  # noqa: E731
+    I = lambda a: a.ctypes.data_as(C.POINTER(C.c_int32))  # noqa: E731
+
+    def up(slot, k, n, sigma=0.02):
+        raw = np.stack([pkg.quantize_row(t, (sigma * rng.standard_normal(k)).astype(np.float32)) for _ in range(n)])
+        assert L.tf_hip_upload_tensor(ctx, slot, t, k, n, raw.ctypes.data, raw.nbytes) == 0
+
+    up(0, d, vocab, 0.5)
+    ones = np.ones(d, np.float32)
+    assert L.tf_hip_upload_tensor(ctx, 1, 0, d, 1, ones.ctypes.data, ones.nbytes) == 0
+    for l in range(layers):
+        s = 16 + 12 * l
+        for slot, k, n in ((1, d, d), (2, d, kv * hd), (3, d, kv * hd), (4, d, d), (9, d, ff), (10, d, ff), (11, ff, d)):
+            up(s + slot, k, n, 2.0 / np.sqrt(k))
+        for slot in (0, 8):
+            assert L.tf_hip_upload_tensor(ctx, s + slot, 0, d, 1, ones.ctypes.data, ones.nbytes) == 0
+    cos, sin = pkg.rope_tables(10000.0, hd, max_seq)
+    assert L.tf_hip_set_rope_table(ctx, F(cos), F(sin), max_seq, hd // 2) == 0
+    prompt = rng.integers(0, vocab, n_prompt).astype(np.int32)
+    res = []
+    for path in (GRAPH, STEP):
+        assert L.tf_hip_set_decode_path(ctx, path) == 0 and L.tf_hip_get_decode_path(ctx) == path
+        assert L.tf_hip_reset(ctx) == 0
+        ids, logits = np.zeros(12, np.int32), np.zeros(vocab, np.float32)
+        assert L.tf_hip_prefill(ctx, I(prompt), n_prompt, None, None) == 0
+        assert L.tf_hip_generate(ctx, 12, I(ids)) == 0
+        assert L.tf_hip_decode(ctx, 3, F(logits), None) == 0
+        rows = [np.zeros((n_prompt + 13, kv, hd), np.float32) for _ in range(2)]
+        for which in (0, 1):
+            assert L.tf_hip_read_kv(ctx, layers - 1, which, 0, n_prompt + 13, F(rows[which])) == 0
+        res.append((ids, logits, *rows))
+    L.tf_hip_destroy(ctx)
+    assert np.array_equal(res[0][0], res[1][0])
+    for a, b in zip(res[0][1:], res[1][1:]):
+        assert rel_err(b, a) <= 1e-5, rel_err(b, a)
+
+
 @pytest.mark.parametrize("n_prompt", [6, 150])
 @pytest.mark.parametrize("preset", ["tiny_mixq4", "tiny_mixfmt"])
 def test_mixed_format_prefill(pkg, gguf, preset, n_prompt):
