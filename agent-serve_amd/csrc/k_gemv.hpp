@@ -14,7 +14,8 @@
 namespace tfk {
 namespace gemv_detail {
 
-constexpr int kStageVec = 9;  // float4 of x per thread: K <= 9 * 4 * kBlock = 9216
+constexpr int kStageVec = 9;  // float4 of x per thread
+static_assert(kStageVec * 4 * kBlock == kGemvMaxK, "the row length this prologue holds");
 
 // x (optionally RMSNorm-ed) and its 16-element partial sums into LDS. Every load of x
 // and of the norm weight is issued before the first one is used, and the prologue ends

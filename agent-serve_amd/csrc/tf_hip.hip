@@ -780,6 +780,67 @@ int prefill_small(tf_hip_ctx* c, int n) {
     return 0;
 }
 
+// The last layer of a prompt after its QKV: nothing reads the output of any row but the last, so
+// attention, wo and the FFN run for that one, as a decode step's kernels do (q: its rotated query
+// row; its residual is row nc - 1 of px; K and V of every row are in the cache). A whole call: 512 tokens of the Llama-3.2-1B
+// shape 4.26 -> 4.08 ms, 333 on its 4-bit weights 3.90 -> 3.75, 2,900 of the Qwen2.5-1.5B shape
+// 30.7 -> 29.6.
+hipError_t prefill_last_row(tf_hip_ctx* c, int l, const float* q, int nc, int pos, int start) {
+    const tf_hip_hparams& p = c->hp;
+    const int D = p.n_embd;
+    auto M = [&](int k) -> const DevMat& { return mat(c, TF_HIP_SLOT_LAYER(l, k)); };
+    hipError_t e = launch_pf_tail(c->ctl, pos, c->hist, c->px + (size_t)(nc - 1) * D, c->x, D, c->st);
+    auto chk = [&](hipError_t r) {
+        if (e == hipSuccess) e = r;
+    };
+    float* kc = c->kc + (size_t)l * c->kv_layer;
+    float* vc = c->vc + (size_t)l * c->kv_layer;
+    if (c->S > 1) {  // the positions split over workgroups
+        AttnArgs a{};
+        a.q = q;
+        a.kc = kc;
+        a.vc = vc;
+        a.rope_cos = c->rope_cos;  // loaded, not applied: q and the cache's keys are rotated
+        a.rope_sin = c->rope_sin;
+        a.part_o = c->part_o;
+        a.part_ml = c->part_ml;
+        a.out = c->att;
+        a.ctl = c->ctl;
+        a.H = p.n_head;
+        a.G = p.n_kv_head;
+        a.hd = p.head_dim;
+        a.max_seq = p.max_seq;
+        a.layout = p.kv_layout;
+        a.S = c->S;
+        a.fixed_pos = pos;
+        a.fixed_start = start;
+        chk(launch_attn_decode(a, c->st));
+    } else {  // at most 512: k_attn_decode would walk them in one workgroup a kv head, 3 us a tile
+        chk(launch_pf_attn(q, c->H + 2 * c->KVd, kc, vc, p.kv_layout, p.n_head, p.n_kv_head, p.head_dim, p.max_seq, 1, pos,
+                           start, c->att, c->H, c->pattn_ws, c->pattn_ws_bytes, c->st));
+    }
+    auto gemv = [&](int kind, const float* x, int K, int mode, float* y, float* tap) {
+        const DevMat& w = M(kind);
+        const int R = pick_rows(w.N);
+        GemvArgs a;
+        a.type = w.type;
+        a.K = K;
+        a.mode = mode;
+        a.x = x;
+        if (mode == GEMV_SILU) {
+            a.norm_w = vec(c, TF_HIP_SLOT_LAYER(l, TF_HIP_LAYER_FFN_NORM));
+            a.eps = p.rms_eps;
+        }
+        add_seg(a, w, y, nullptr, tap, R);
+        if (mode == GEMV_SILU) a.seg[0].b = M(TF_HIP_LAYER_UP);
+        chk(launch_gemv(a, R, c->st));
+    };
+    gemv(TF_HIP_LAYER_O, c->att, c->H, GEMV_RESID, c->x, nullptr);
+    gemv(TF_HIP_LAYER_GATE, c->x, D, GEMV_SILU, c->h, nullptr);
+    gemv(TF_HIP_LAYER_DOWN, c->h, p.n_ff, GEMV_RESID, c->x, c->taps + (size_t)l * D);
+    return e;
+}
+
 // n prompt tokens, staged at hist[c->pos ..], through the matrix-core layers in chunks
 // of pf_cap rows; attention of every chunk covers the prompt from c->pos (the reference
 // attends within the prefill call only, attention.cpp:82-111). Ends with the lm_head of
@@ -788,6 +849,7 @@ int prefill_mfma(tf_hip_ctx* c, int n) {
     const tf_hip_hparams& p = c->hp;
     const int D = p.n_embd, F = p.n_ff, Hd = c->H, KVd = c->KVd, NQ = Hd + 2 * KVd;
     const int start = c->pos;
+    const bool last_row = std::max(std::max(D, F), Hd) <= kGemvMaxK;
     hipError_t e = hipSuccess;
     auto chk = [&](hipError_t r) {
         if (e == hipSuccess) e = r;
@@ -875,6 +937,10 @@ int prefill_mfma(tf_hip_ctx* c, int n) {
                     chk(launch_pf_rope_store(c->pqkv, NQ, nc, p.n_head, p.n_kv_head, p.head_dim, c->rope_cos,
                                              c->rope_sin, pos0, kc, vc, p.kv_layout, p.max_seq, c->st));
             }
+            if (l + 1 == p.n_layer && last_row) {
+                if (last) chk(prefill_last_row(c, l, c->pqkv + (int64_t)(nc - 1) * NQ, nc, start + n - 1, start));
+                continue;
+            }
             chk(launch_pf_attn(c->pqkv, NQ, kc, vc, p.kv_layout, p.n_head, p.n_kv_head, p.head_dim, p.max_seq, nc,
                                pos0, start, c->patt, Hd, c->pattn_ws, c->pattn_ws_bytes, c->st));
             chk(launch_pf_split(c->patt, Hd, nullptr, 0.0f, Hd, nc, Mpad, c->pxa, c->prs, c->st));
@@ -940,7 +1006,7 @@ int prefill_mfma(tf_hip_ctx* c, int n) {
             }
         }
     }
-    chk(launch_pf_tail(c->ctl, start + n - 1, c->hist, c->px + (size_t)(nc - 1) * D, c->x, D, c->st));
+    if (!last_row) chk(launch_pf_tail(c->ctl, start + n - 1, c->hist, c->px + (size_t)(nc - 1) * D, c->x, D, c->st));
     chk(launch_lm_head(c));
     if (e != hipSuccess) return fail(c, TF_HIP_EDEVICE, std::string("prefill launch: ") + hipGetErrorString(e));
     return 0;
