@@ -12,6 +12,8 @@
 // round each instead of a few walking tiles one after the other.
 // No workgroup waits on another inside a launch: on this multi-XCD part a device-scope
 // fence writes back the XCD's L2, which costs more than the kernel boundary.
+#include <algorithm>
+
 #include "dev_common.hpp"
 #include "tf_internal.hpp"
 
@@ -50,14 +52,18 @@ __device__ __forceinline__ Split split_of(const AttnArgs& a) {
     return sp;
 }
 
-template <int HDM>
+// EXACT: head_dim is HDM itself, known to the compiler (no divisions, loops unrolled). Bound by
+// its chain of memory round, scores, softmax and P.V on a tile a workgroup: 32 x 64 heads over
+// 8, 1,000 of 4,096 positions, 10.5 us before this and the two threads a score, 6.4 now (a fifth
+// of it the launch of workgroups past the positions); k_attn_combine 5.0 -> 3.3.
+template <int HDM, bool EXACT>
 __global__ __launch_bounds__(kBlock) void k_attn_decode(const AttnArgs a) {
     constexpr int kMaxPairs = AttnShape<HDM>::kPairs;
     constexpr int kQPairs = AttnShape<HDM>::kQPairs;
     constexpr int kTileVec = AttnShape<HDM>::kTileVec;
     const int g = blockIdx.x / a.S;
     const int s = blockIdx.x % a.S;
-    const int hd = a.hd, d2 = hd / 2, hd4 = hd / 4;
+    const int hd = EXACT ? HDM : a.hd, d2 = hd / 2, hd4 = hd / 4;
     const int n_rep = a.H / a.G;
     const Split sp = split_of(a);
     if (s >= sp.n_act) return;
@@ -173,25 +179,24 @@ __global__ __launch_bounds__(kBlock) void k_attn_decode(const AttnArgs a) {
             }
         }
         __syncthreads();
-        // scores in the order of dot_f32 (8 lanes over i = 0, 8, ..., then hsum8; quant.cpp:198-214)
-        for (int i = tid; i < n_rep * tn; i += kBlock) {
-            const int r = i / tn, j = i % tn;
-            const float* qr = qs + r * hd;
-            const float* krow = kt + j * ks;
-            float c[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        // scores in the order of dot_f32 (8 lanes over i = 0, 8, ..., then hsum8; quant.cpp:198-214),
+        // two threads a score: lanes 0..3 and 4..7, added pairwise across the two
+        for (int i = tid; i < n_rep * kAttnTile * 2; i += kBlock) {
+            const int half = i & 1, r = i / (2 * kAttnTile), j = i / 2 % kAttnTile;
+            const float* qr = qs + r * hd + 4 * half;
+            const float* krow = kt + (j < tn ? j : 0) * ks + 4 * half;
+            float c[4] = {0, 0, 0, 0};
+#pragma unroll 8
             for (int e = 0; e < hd; e += 8) {
-                const float4 q0 = *(const float4*)(qr + e), q1 = *(const float4*)(qr + e + 4);
-                const float4 x0 = *(const float4*)(krow + e), x1 = *(const float4*)(krow + e + 4);
+                const float4 q0 = *(const float4*)(qr + e), x0 = *(const float4*)(krow + e);
                 c[0] = fmaf(q0.x, x0.x, c[0]);
                 c[1] = fmaf(q0.y, x0.y, c[1]);
                 c[2] = fmaf(q0.z, x0.z, c[2]);
                 c[3] = fmaf(q0.w, x0.w, c[3]);
-                c[4] = fmaf(q1.x, x1.x, c[4]);
-                c[5] = fmaf(q1.y, x1.y, c[5]);
-                c[6] = fmaf(q1.z, x1.z, c[6]);
-                c[7] = fmaf(q1.w, x1.w, c[7]);
             }
-            pr[r * kAttnTile + j] = scale * (((c[0] + c[4]) + (c[1] + c[5])) + ((c[2] + c[6]) + (c[3] + c[7])));
+#pragma unroll
+            for (int k = 0; k < 4; ++k) c[k] += dpp<kDppXor1>(c[k]);
+            if (half == 0 && j < tn) pr[r * kAttnTile + j] = scale * ((c[0] + c[1]) + (c[2] + c[3]));
         }
         __syncthreads();
         // online softmax statistics: wave w handles heads r = w, w + 4, ...
@@ -218,6 +223,7 @@ __global__ __launch_bounds__(kBlock) void k_attn_decode(const AttnArgs a) {
             if (pi < n_rep * hd) {
                 const int r = pi / hd, d = pi % hd;
                 float o = o_acc[k] * st[3 * r + 2];
+#pragma unroll 8
                 for (int j = 0; j < tn; ++j) o = fmaf(pr[r * kAttnTile + j], vt[j * hd + d], o);
                 o_acc[k] = o;
             }
@@ -256,46 +262,56 @@ __global__ __launch_bounds__(kBlock) void k_attn_decode(const AttnArgs a) {
 // the groups are added in group order (a fixed order for a given split count).
 constexpr int kCombThreads = 1024;
 
+template <int HD>
 __global__ __launch_bounds__(kCombThreads) void k_attn_combine(const AttnArgs a) {
     const Split sp = split_of(a);
     if (sp.n_act <= 1) return;  // k_attn_decode wrote the output
     __shared__ float w[kAttnMaxSplits];
-    __shared__ float red[kCombThreads / kWave];
+    __shared__ float red[2][kCombThreads / kWave];
     __shared__ float part[kCombThreads];
-    const int h = blockIdx.x, n = sp.n_act, hd = a.hd;
+    const int h = blockIdx.x, n = sp.n_act, hd = HD ? HD : a.hd;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const float* ml = a.part_ml + (int64_t)h * a.S * 2;
-    float m = -INFINITY;
-    for (int t = tid; t < n; t += kCombThreads) m = fmaxf(m, ml[2 * t]);
-    m = wave_max(m);
-    if (lane == 0) red[wave] = m;
-    __syncthreads();
-    float M = red[0];
-    for (int i = 1; i < kCombThreads / kWave; ++i) M = fmaxf(M, red[i]);
-    __syncthreads();  // red is reused below
-    float l = 0.0f;
-    for (int t = tid; t < n; t += kCombThreads) {
-        const float wt = expf(ml[2 * t] - M);
-        w[t] = wt;
-        l = fmaf(ml[2 * t + 1], wt, l);
-    }
-    l = wave_sum(l);
-    if (lane == 0) red[wave] = l;
-    __syncthreads();
-    float L = 0.0f;
-    for (int i = 0; i < kCombThreads / kWave; ++i) L += red[i];
     const int groups = kCombThreads / hd;
     const int d = tid % hd, grp = tid / hd;
+    const float* po = a.part_o + (int64_t)h * a.S * hd + d;
+    // one memory round: this thread's (m, l) and its first partials
+    static_assert(kAttnMaxSplits <= kCombThreads, "a split per thread");
+    constexpr int kFirst = 4;
+    const float m_t = tid < n ? ml[2 * tid] : -INFINITY, l_t = tid < n ? ml[2 * tid + 1] : 0.0f;
+    float first[kFirst];
+#pragma unroll
+    for (int i = 0; i < kFirst; ++i) {
+        const int t = grp + i * groups;
+        first[i] = po[(int64_t)(t < n ? t : n - 1) * hd];
+    }
+    float M = wave_max(m_t);
+    if (lane == 0) red[0][wave] = M;
+    __syncthreads();
+    M = red[0][0];
+#pragma unroll
+    for (int i = 1; i < kCombThreads / kWave; ++i) M = fmaxf(M, red[0][i]);
+    const float wt = tid < n ? expf(m_t - M) : 0.0f;
+    if (tid < n) w[tid] = wt;
+    const float l = wave_sum(l_t * wt);
+    if (lane == 0) red[1][wave] = l;
+    __syncthreads();
+    float L = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kCombThreads / kWave; ++i) L += red[1][i];
     float o = 0.0f;
     if (grp < groups) {
-        const float* po = a.part_o + (int64_t)h * a.S * hd + d;
+#pragma unroll
+        for (int i = 0; i < kFirst; ++i)
+            if (grp + i * groups < n) o = fmaf(first[i], w[grp + i * groups], o);
 #pragma unroll 8
-        for (int t = grp; t < n; t += groups) o = fmaf(po[(int64_t)t * hd], w[t], o);
+        for (int t = grp + kFirst * groups; t < n; t += groups) o = fmaf(po[(int64_t)t * hd], w[t], o);
     }
     part[tid] = o;
     __syncthreads();
     if (tid < hd) {
         float sum = 0.0f;
+#pragma unroll 8
         for (int g = 0; g < groups; ++g) sum += part[g * hd + tid];
         a.out[(int64_t)h * hd + tid] = sum / L;
     }
@@ -309,20 +325,34 @@ int attn_splits(int max_seq) {
     return s < 2 ? 2 : (s > kAttnMaxSplits ? kAttnMaxSplits : s);
 }
 
-hipError_t launch_attn_decode(const AttnArgs& a, hipStream_t st) {
+hipError_t launch_attn_decode(const AttnArgs& args, hipStream_t st) {
+    AttnArgs a = args;
+    if (a.hd > kCombThreads) return hipErrorInvalidValue;
+    // a known position: only the splits it fills (split_of's cut of the same positions does not
+    // change; a 4096-position cache would launch 128 workgroups a kv head for 32 with work)
+    if (a.fixed_pos >= 0) a.S = std::min(a.S, (a.fixed_pos + 1 - a.fixed_start + kAttnMinChunk - 1) / kAttnMinChunk);
     const int n_rep = a.H / a.G;
     const size_t lds = sizeof(float) * ((size_t)n_rep * a.hd + 2 * (size_t)a.hd + (size_t)kAttnTile * (a.hd + 4) +
                                         (size_t)kAttnTile * a.hd + (size_t)n_rep * kAttnTile + 3 * (size_t)n_rep);
-    if (a.hd <= 64)
-        hipLaunchKernelGGL(k_attn_decode<64>, dim3(a.G * a.S), dim3(kBlock), lds, st, a);
+    const dim3 grid((unsigned)(a.G * a.S));
+    if (a.hd == 64)
+        hipLaunchKernelGGL((k_attn_decode<64, true>), grid, dim3(kBlock), lds, st, a);
+    else if (a.hd == 128)
+        hipLaunchKernelGGL((k_attn_decode<128, true>), grid, dim3(kBlock), lds, st, a);
+    else if (a.hd <= 64)
+        hipLaunchKernelGGL((k_attn_decode<64, false>), grid, dim3(kBlock), lds, st, a);
     else if (a.hd <= 128)
-        hipLaunchKernelGGL(k_attn_decode<128>, dim3(a.G * a.S), dim3(kBlock), lds, st, a);
+        hipLaunchKernelGGL((k_attn_decode<128, false>), grid, dim3(kBlock), lds, st, a);
     else
-        hipLaunchKernelGGL(k_attn_decode<256>, dim3(a.G * a.S), dim3(kBlock), lds, st, a);
-    hipError_t e = hipGetLastError();
+        hipLaunchKernelGGL((k_attn_decode<256, false>), grid, dim3(kBlock), lds, st, a);
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.S == 1) return e;
-    if (a.hd > kCombThreads) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_attn_combine, dim3(a.H), dim3(kCombThreads), 0, st, a);
+    if (a.hd == 64)
+        hipLaunchKernelGGL(k_attn_combine<64>, dim3(a.H), dim3(kCombThreads), 0, st, a);
+    else if (a.hd == 128)
+        hipLaunchKernelGGL(k_attn_combine<128>, dim3(a.H), dim3(kCombThreads), 0, st, a);
+    else
+        hipLaunchKernelGGL(k_attn_combine<0>, dim3(a.H), dim3(kCombThreads), 0, st, a);
     return hipGetLastError();
 }
 
