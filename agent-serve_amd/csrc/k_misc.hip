@@ -3,6 +3,8 @@
 #include <mutex>
 #include <vector>
 
+#include <algorithm>
+
 #include "formats.hpp"
 
 namespace tfk {
@@ -152,6 +154,38 @@ __global__ __launch_bounds__(kBlock) void k_rope_rows(float* x, int64_t n_pairs,
     }
 }
 
+// A call's inputs: its tokens (up to kStageTokens, by value) at hist[pos ..], att_start and mode.
+// One launch where two or three small host-to-device copies each cost a copy engine's round trip
+// (about 8 us of a call's 40 beyond its kernels).
+__global__ void k_stage(Ctl* ctl, int32_t* hist, StageTokens t, int n, int pos, int att_start, int mode) {
+    if ((int)threadIdx.x < n) hist[pos + threadIdx.x] = t.tok[threadIdx.x];
+    if (threadIdx.x == 0) {
+        ctl->att_start = att_start;
+        ctl->mode = mode;
+    }
+}
+
+// A call's results into pinned host memory: the control block and hist[pos .. pos + n).
+__global__ __launch_bounds__(kBlock) void k_report(const Ctl* ctl, Ctl* host_ctl, const int32_t* hist, int pos, int n,
+                                                   int32_t* host_tok) {
+    for (int i = threadIdx.x; i < n; i += kBlock) host_tok[i] = hist[pos + i];
+    if (threadIdx.x == 0) *host_ctl = *ctl;
+}
+
+// KV cache and control block of a reset context, n4 16-byte words in each cache.
+__global__ __launch_bounds__(kBlock) void k_reset(float4* kc, float4* vc, size_t n4, Ctl* ctl, uint32_t epoch) {
+    const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < n4; i += (size_t)gridDim.x * kBlock) {
+        kc[i] = z;
+        vc[i] = z;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        Ctl c = {};
+        c.epoch = epoch;
+        *ctl = c;
+    }
+}
+
 __global__ __launch_bounds__(kBlock) void k_argmax(const float* x, int n, Ctl* ctl) {
     __shared__ unsigned long long wb[kWavesPerBlock];
     unsigned long long best = 0;
@@ -268,6 +302,28 @@ hipError_t launch_rope_rows(float* x, int seq, int n_heads, int hd, int pos0, co
 
 hipError_t launch_argmax(const float* x, int n, Ctl* ctl, hipStream_t st) {
     hipLaunchKernelGGL(k_argmax, dim3(grid_for(n)), dim3(kBlock), 0, st, x, n, ctl);
+    return hipGetLastError();
+}
+
+hipError_t launch_stage(Ctl* ctl, int32_t* hist, const int32_t* tokens, int n, int pos, int att_start, int mode,
+                        hipStream_t st) {
+    if (n < 0 || n > kStageTokens) return hipErrorInvalidValue;
+    StageTokens t{};
+    for (int i = 0; i < n; ++i) t.tok[i] = tokens[i];
+    hipLaunchKernelGGL(k_stage, dim3(1), dim3(kWave), 0, st, ctl, hist, t, n, pos, att_start, mode);
+    return hipGetLastError();
+}
+
+hipError_t launch_report(const Ctl* ctl, Ctl* host_ctl, const int32_t* hist, int pos, int n, int32_t* host_tok,
+                         hipStream_t st) {
+    hipLaunchKernelGGL(k_report, dim3(1), dim3(kBlock), 0, st, ctl, host_ctl, hist, pos, n, host_tok);
+    return hipGetLastError();
+}
+
+hipError_t launch_reset(float* kc, float* vc, size_t n, Ctl* ctl, uint32_t epoch, hipStream_t st) {
+    if (n % 4 != 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_reset, dim3((unsigned)std::min<size_t>((n / 4 + kBlock - 1) / kBlock, 8 * (size_t)device_cu_count())),
+                       dim3(kBlock), 0, st, (float4*)kc, (float4*)vc, n / 4, ctl, epoch);
     return hipGetLastError();
 }
 

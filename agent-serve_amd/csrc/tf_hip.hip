@@ -66,7 +66,7 @@ struct tf_hip_ctx {
     bool have_logits = false;
     void* sample_work = nullptr;      // tf_hip_sample: sort buffers, probabilities, radix-sort scratch
     size_t sample_bytes = 0;
-    int32_t* d_sampled = nullptr;     // the sampled token
+    int32_t* d_sampled = nullptr;     // the sampled token (pinned host memory)
     Ctl* sample_ctl = nullptr;        // argmax of a greedy tf_hip_sample
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
@@ -600,12 +600,14 @@ int run_step(tf_hip_ctx* c, int n, int greedy, int lm_every, int att_start) {
     return 0;
 }
 
-// Writes att_start and mode of the device control block.
-int set_ctl(tf_hip_ctx* c, int att_start, int mode) {
-    c->ctl_host->att_start = att_start;
-    c->ctl_host->mode = mode;
-    HIPCHK(c, hipMemcpyAsync((char*)c->ctl + offsetof(Ctl, att_start), (char*)c->ctl_host + offsetof(Ctl, att_start),
-                             2 * sizeof(int32_t), hipMemcpyHostToDevice, c->st));
+// Tokens tokens[0..n) at hist[c->pos ..], att_start and mode of the device control block.
+int stage_call(tf_hip_ctx* c, const int32_t* tokens, int n, int att_start, int mode) {
+    const bool copy = n > kStageTokens;
+    if (copy) {
+        std::memcpy(c->tok_host, tokens, (size_t)n * 4);
+        HIPCHK(c, hipMemcpyAsync(c->hist + c->pos, c->tok_host, (size_t)n * 4, hipMemcpyHostToDevice, c->st));
+    }
+    HIPCHK(c, launch_stage(c->ctl, c->hist, tokens, copy ? 0 : n, c->pos, att_start, mode, c->st));
     return 0;
 }
 
@@ -1012,10 +1014,11 @@ int prefill_mfma(tf_hip_ctx* c, int n) {
     return 0;
 }
 
-int finish_step_outputs(tf_hip_ctx* c, float* logits, int32_t* argmax) {
+// Waits for the call; n_hist tokens from hist[pos0] arrive in tok_host.
+int finish_step_outputs(tf_hip_ctx* c, float* logits, int32_t* argmax, int pos0 = 0, int n_hist = 0) {
+    HIPCHK(c, launch_report(c->ctl, c->ctl_host, c->hist, pos0, n_hist, c->tok_host, c->st));
     if (logits)
         HIPCHK(c, hipMemcpyAsync(logits, c->logits, (size_t)c->hp.n_vocab * 4, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipMemcpyAsync(c->ctl_host, c->ctl, sizeof(Ctl), hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
     if (c->ctl_host->err == 2) return fail(c, TF_HIP_EDEVICE, "step kernel: an exchange wait timed out");
     if (c->ctl_host->err) return fail(c, TF_HIP_EDEVICE, "device reported an invalid token");
@@ -1115,6 +1118,7 @@ int tf_hip_destroy(tf_hip_ctx* c) {
     for (void* p : c->allocs) (void)hipFree(p);
     if (c->ctl_host) (void)hipHostFree(c->ctl_host);
     if (c->tok_host) (void)hipHostFree(c->tok_host);
+    if (c->d_sampled) (void)hipHostFree(c->d_sampled);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->st) (void)hipStreamDestroy(c->st);
@@ -1226,11 +1230,8 @@ int tf_hip_reset(tf_hip_ctx* c) {
     HIPCHK(c, hipStreamSynchronize(c->st));
     c->pos = 0;
     c->have_logits = false;
-    std::memset(c->ctl_host, 0, sizeof(Ctl));
-    c->ctl_host->epoch = c->epoch;  // exchange words keep old epochs: never reuse one
-    HIPCHK(c, hipMemcpyAsync(c->ctl, c->ctl_host, sizeof(Ctl), hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, hipMemsetAsync(c->kc, 0, c->kv_layer * c->hp.n_layer * 4, c->st));
-    HIPCHK(c, hipMemsetAsync(c->vc, 0, c->kv_layer * c->hp.n_layer * 4, c->st));
+    // exchange words keep old epochs: never reuse one
+    HIPCHK(c, launch_reset(c->kc, c->vc, c->kv_layer * c->hp.n_layer, c->ctl, c->epoch, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
     return 0;
 }
@@ -1247,9 +1248,7 @@ int tf_hip_decode(tf_hip_ctx* c, int32_t token, float* logits, int32_t* argmax) 
     if (use_step < 0) return use_step;
     int rc = use_step ? 0 : ensure_graph(c);
     if (rc) return rc;
-    c->tok_host[0] = token;
-    HIPCHK(c, hipMemcpyAsync(c->hist + c->pos, c->tok_host, 4, hipMemcpyHostToDevice, c->st));
-    if ((rc = set_ctl(c, 0, 0))) return rc;
+    if ((rc = stage_call(c, &token, 1, 0, 0))) return rc;
     if ((rc = run_tokens(c, &use_step, 1, 0, 1, 0))) return rc;
     c->pos += 1;
     rc = finish_step_outputs(c, logits, argmax);
@@ -1273,9 +1272,7 @@ int tf_hip_prefill(tf_hip_ctx* c, const int32_t* tokens, int32_t n, float* logit
     if (use_step < 0) return use_step;
     int rc = (use_pf || use_step) ? 0 : ensure_graph(c);
     if (rc) return rc;
-    std::memcpy(c->tok_host, tokens, (size_t)n * 4);
-    HIPCHK(c, hipMemcpyAsync(c->hist + c->pos, c->tok_host, (size_t)n * 4, hipMemcpyHostToDevice, c->st));
-    if ((rc = set_ctl(c, c->pos, 0))) return rc;
+    if ((rc = stage_call(c, tokens, n, c->pos, 0))) return rc;
     HIPCHK(c, hipEventRecord(c->ev0, c->st));
     if (use_pf) {
         if ((rc = n <= kPfSmallRows && c->pf_small ? prefill_small(c, n) : prefill_mfma(c, n))) return rc;
@@ -1304,13 +1301,12 @@ int tf_hip_generate(tf_hip_ctx* c, int32_t n, int32_t* out) {
     int rc = use_step ? 0 : ensure_graph(c);
     if (rc) return rc;
     const int pos0 = c->pos;
-    if ((rc = set_ctl(c, 0, 1))) return rc;
+    if ((rc = stage_call(c, nullptr, 0, 0, 1))) return rc;
     HIPCHK(c, hipEventRecord(c->ev0, c->st));
     if ((rc = run_tokens(c, &use_step, n, 1, 1, 0))) return rc;
     HIPCHK(c, hipEventRecord(c->ev1, c->st));
-    HIPCHK(c, hipMemcpyAsync(c->tok_host, c->hist + pos0, (size_t)n * 4, hipMemcpyDeviceToHost, c->st));
     c->pos += n;
-    rc = finish_step_outputs(c, nullptr, nullptr);
+    rc = finish_step_outputs(c, nullptr, nullptr, pos0, n);
     if (rc) return rc;
     std::memcpy(out, c->tok_host, (size_t)n * 4);
     HIPCHK(c, hipEventElapsedTime(&c->last_ms, c->ev0, c->ev1));
@@ -1454,15 +1450,14 @@ int tf_hip_profile_generate(tf_hip_ctx* c, int32_t n, int32_t* out, float* ms_by
     int rc = check_ready(c);
     if (rc) return rc;
     const int pos0 = c->pos;
-    if ((rc = set_ctl(c, 0, 1))) return rc;
+    if ((rc = stage_call(c, nullptr, 0, 0, 1))) return rc;
     Prof prof;
     for (int i = 0; i < n; ++i) {
         const hipError_t e = enqueue_step(c, &prof, pos0 + i, 0);
         if (e != hipSuccess) return fail(c, TF_HIP_EDEVICE, std::string("profile step: ") + hipGetErrorString(e));
     }
-    HIPCHK(c, hipMemcpyAsync(c->tok_host, c->hist + pos0, (size_t)n * 4, hipMemcpyDeviceToHost, c->st));
     c->pos += n;
-    rc = finish_step_outputs(c, nullptr, nullptr);
+    rc = finish_step_outputs(c, nullptr, nullptr, pos0, n);
     if (rc) return rc;
     std::memcpy(out, c->tok_host, (size_t)n * 4);
     for (int k = 0; k < kNumClasses; ++k) {
@@ -1820,9 +1815,9 @@ int tf_hip_sample(tf_hip_ctx* c, float temperature, float top_p, float r, int32_
     int rc;
     if (!c->d_sampled) {
         const size_t bytes = sample_work_bytes(V);
-        if ((rc = dalloc(c, (uint8_t**)&c->sample_work, bytes)) || (rc = dalloc(c, &c->d_sampled, 64)) ||
-            (rc = dalloc(c, &c->sample_ctl, sizeof(Ctl))))
+        if ((rc = dalloc(c, (uint8_t**)&c->sample_work, bytes)) || (rc = dalloc(c, &c->sample_ctl, sizeof(Ctl))))
             return rc;
+        HIPCHK(c, hipHostMalloc((void**)&c->d_sampled, 64, 0));
         c->sample_bytes = bytes;
     }
     int32_t tok = 0;
@@ -1841,9 +1836,8 @@ int tf_hip_sample(tf_hip_ctx* c, float temperature, float top_p, float r, int32_
                                             c->d_sampled, nullptr, nullptr, c->st)
                             : launch_sample_top(c->logits, V, temperature, top_p, r, c->sample_work, c->sample_bytes,
                                                 c->d_sampled, c->st));
-            HIPCHK(c, hipMemcpyAsync(c->tok_host, c->d_sampled, 4, hipMemcpyDeviceToHost, c->st));
             HIPCHK(c, hipStreamSynchronize(c->st));
-            tok = c->tok_host[0];
+            tok = *c->d_sampled;
             if (tok >= 0) break;
         }
     }

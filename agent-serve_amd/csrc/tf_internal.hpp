@@ -324,6 +324,18 @@ hipError_t launch_sample_top(const float* logits, int n, float temperature, floa
 hipError_t launch_rope_rows(float* x, int seq, int n_heads, int hd, int pos0, const float* cos_tab,
                             const float* sin_tab, hipStream_t st);
 hipError_t launch_argmax(const float* x, int n, Ctl* ctl, hipStream_t st);
+// A call's inputs and results without copy engines (k_misc.hip): up to kStageTokens tokens at
+// hist[pos ..] with att_start and mode; the control block and n tokens from hist[pos] into pinned
+// host memory; a reset context's caches (n floats each) and control block.
+constexpr int kStageTokens = 64;
+struct StageTokens {
+    int32_t tok[kStageTokens];
+};
+hipError_t launch_stage(Ctl* ctl, int32_t* hist, const int32_t* tokens, int n, int pos, int att_start, int mode,
+                        hipStream_t st);
+hipError_t launch_report(const Ctl* ctl, Ctl* host_ctl, const int32_t* hist, int pos, int n, int32_t* host_tok,
+                         hipStream_t st);
+hipError_t launch_reset(float* kc, float* vc, size_t n, Ctl* ctl, uint32_t epoch, hipStream_t st);
 // The read and copy streams (k_misc.hip): buffers filled by launch_fill_stream hold 32-bit
 // word i = i * kStreamMul, and k_read_stream writes one integer partial sum per wave.
 constexpr uint32_t kStreamMul = 0x9E3779B1u;
