@@ -70,6 +70,32 @@ __global__ __launch_bounds__(kBlock) void k_dequant_rows(const DevMat m, int64_t
     }
 }
 
+// A wave per row.
+template <int T>
+__global__ __launch_bounds__(kBlock) void k_row_norm_max(const DevMat m, float* out) {
+    using F = Fmt<T>;
+    const int steps = (int)(m.K / F::E), lane = threadIdx.x & 63;
+    float best = 0.0f;
+    for (int64_t r = (int64_t)blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6); r < m.N; r += (int64_t)gridDim.x * kWavesPerBlock) {
+        float ss = 0.0f;
+        for (int s = lane; s < steps; s += kWave) {
+            float v[F::E];
+            F::dequant(F::load(F::row(m, r), s), v);
+#pragma unroll
+            for (int j = 0; j < F::E; ++j) ss = fmaf(v[j], v[j], ss);
+        }
+        best = fmaxf(best, wave_sum(ss));
+    }
+    __shared__ float wb[kWavesPerBlock];
+    if (lane == 0) wb[threadIdx.x >> 6] = best;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int i = 1; i < kWavesPerBlock; ++i) best = fmaxf(best, wb[i]);
+        // positive floats order as their bits; 1.001 covers the sum's and the root's rounding
+        atomicMax((int*)out, __float_as_int(sqrtf(best) * 1.001f));
+    }
+}
+
 // GGUF rows -> DevMat streams. One thread per GGUF block (Q6_K: per 32-element group).
 __global__ __launch_bounds__(kBlock) void k_repack(int type, const uint8_t* raw, int64_t K, int64_t N, DevMat m) {
     const int64_t nb = K / 32;  // 32-element groups per row
@@ -279,6 +305,13 @@ hipError_t launch_dequant_rows(const DevMat& m, int64_t row0, int64_t nrows, flo
     const int64_t steps = m.K / fmt_step_elems(m.type);
     const int blocks = grid_for(nrows * steps);
     TF_DISPATCH_TYPE(m.type, hipLaunchKernelGGL((k_dequant_rows<T_>), dim3(blocks), dim3(kBlock), 0, st, m, row0, nrows, out));
+    return hipGetLastError();
+}
+
+hipError_t launch_row_norm_max(const DevMat& m, float* out, hipStream_t st) {
+    // two workgroups a CU: an atomic each, and 8,192 of them on one word took 150 us
+    const int blocks = (int)std::min<int64_t>((m.N + kWavesPerBlock - 1) / kWavesPerBlock, 2 * (int64_t)device_cu_count());
+    TF_DISPATCH_TYPE(m.type, hipLaunchKernelGGL((k_row_norm_max<T_>), dim3(blocks), dim3(kBlock), 0, st, m, out));
     return hipGetLastError();
 }
 

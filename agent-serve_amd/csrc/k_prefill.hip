@@ -202,10 +202,12 @@ constexpr int kSplitGroups = 8;  // 8-element groups per thread: rows up to 256 
 
 // The split of row m whose values thread tid holds as v[i] = 8-element group tid + i ST
 // (ST = 64 WPR threads per row; groups past K / 8 hold clamped re-reads, masked here):
-// rmsnorm with weight w when given, the power-of-two scale, hi + lo into the fragments.
+// rmsnorm with weight w when given, the power-of-two scale, hi + lo into the fragments; the sum
+// of squares of what was split into xn[m] when given.
 template <int NG, int WPR>
 __device__ __forceinline__ void split_emit(float (&v)[NG][8], int tid, int m, int K, const float* w, float eps,
-                                           h8_t* xa, float* rs, double* red_d, float* red_f) {
+                                           h8_t* xa, float* rs, float* xn, double* red_d, float* red_f,
+                                           float* red_s) {
     constexpr int ST = 64 * WPR;
     const int ng = K / 8, nblk = K / 32;
     h8_t* tile = xa + (int64_t)(m / 16) * nblk * 128 + (m % 16);
@@ -235,18 +237,27 @@ __device__ __forceinline__ void split_emit(float (&v)[NG][8], int tid, int m, in
             for (int e = 0; e < 8; ++e) v[i][e] = v[i][e] * inv * g[e];
         }
     }
-    float amax = 0.0f;
+    float amax = 0.0f, sq = 0.0f;
 #pragma unroll
     for (int i = 0; i < NG; ++i)
         if (tid + i * ST < ng)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(v[i][e]));
+            for (int e = 0; e < 8; ++e) {
+                amax = fmaxf(amax, fabsf(v[i][e]));
+                sq = fmaf(v[i][e], v[i][e], sq);
+            }
     amax = wave_max(amax);
+    if (xn) sq = wave_sum(sq);
     if (WPR > 1) {
-        if ((tid & 63) == 0) red_f[tid >> 6] = amax;
+        if ((tid & 63) == 0) {
+            red_f[tid >> 6] = amax;
+            red_s[tid >> 6] = sq;
+        }
         __syncthreads();
         amax = fmaxf(fmaxf(red_f[0], red_f[1]), fmaxf(red_f[2], red_f[3]));
+        sq = (red_s[0] + red_s[1]) + (red_s[2] + red_s[3]);
     }
+    if (xn && tid == 0) xn[m] = sq;
     int ex = 0;
     (void)frexpf(amax, &ex);  // amax = f 2^ex, f in [0.5, 1)
     int e2 = amax > 0.0f ? 15 - ex : 0;
@@ -294,10 +305,10 @@ __device__ __forceinline__ void split_zero(int tid, int m, int K, h8_t* xa, floa
 // workgroup fill whole 64-byte lines of a fragment). Rows M.. are zeros with rs = 0.
 template <int NG, int WPR>
 __global__ __launch_bounds__(kBlock) void k_pf_split(const float* x, int64_t ldx, const float* w, float eps, int K,
-                                                     int M, h8_t* xa, float* rs) {
+                                                     int M, h8_t* xa, float* rs, float* xn) {
     constexpr int ST = 64 * WPR;  // threads per row
     __shared__ double red_d[kWavesPerBlock];
-    __shared__ float red_f[kWavesPerBlock];
+    __shared__ float red_f[kWavesPerBlock], red_s[kWavesPerBlock];
     const int m = WPR == 1 ? blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6) : blockIdx.x;
     const int tid = WPR == 1 ? threadIdx.x & 63 : threadIdx.x;
     const int ng = K / 8;
@@ -315,13 +326,37 @@ __global__ __launch_bounds__(kBlock) void k_pf_split(const float* x, int64_t ldx
         v[i][0] = a.x; v[i][1] = a.y; v[i][2] = a.z; v[i][3] = a.w;
         v[i][4] = b.x; v[i][5] = b.y; v[i][6] = b.z; v[i][7] = b.w;
     }
-    split_emit<NG, WPR>(v, tid, m, K, w, eps, xa, rs, red_d, red_f);
+    split_emit<NG, WPR>(v, tid, m, K, w, eps, xa, rs, xn, red_d, red_f, red_s);
 }
 
 // ---------------------------------------------------------------- GEMM
 
 // Field of the segment holding output subtile u (uniform per wave: scalar selects).
 #define PF_SEL(s, f) ((s) == 0 ? a.seg[0].f : ((s) == 1 ? a.seg[1].f : a.seg[2].f))
+
+// Hidden rows as the next GEMM's operand: h = silu(g) u with |g| and |u| at most the
+// row's norm times the largest norm of a gate / up row, so |h| < 2^hid_exp without a pass over the
+// row, which no workgroup has whole. The operand's power of two comes from that bound instead
+// of the row's largest value: fp16's pair then keeps 22 bits of every value down to 2^-18 of the
+// bound, and 2^-40 of the bound below that. The bound is 2^7 to 2^9 above the row's largest value
+// for N(0, sigma) weights; one 2^14 above would still leave errors at 2^-26 of it. (Written as fp32
+// rows and split in a pass of their own, 11.7 us a layer at 512 rows of 8,192: a whole 512-token
+// prompt of the Llama-3.2-1B shape 4.10 -> 3.87 ms, 2,900 tokens of the Qwen2.5-1.5B shape 29.6 ->
+// 27.9, 333 on 4-bit weights 3.75 -> 3.54.)
+__device__ __forceinline__ int hid_exp(const PfGemmArgs& a, int row) {
+    int ex, eg, eu;
+    (void)frexpf(a.xn[row], &ex);
+    (void)frexpf(*a.wn_gate, &eg);
+    (void)frexpf(*a.wn_up, &eu);
+    const int e = 15 - (ex + eg + eu);
+    return e < -100 ? -100 : (e > 100 ? 100 : e);
+}
+// Element (row, col) of the operand: its hi half; the lo half 512 halves on.
+__device__ __forceinline__ _Float16* hid_at(const PfGemmArgs& a, int row, int col) {
+    col += a.hid_col0;
+    return (_Float16*)a.hid + (((int64_t)(row / 16) * a.hid_nblk + col / 32) * 128 + row % 16 + 16 * (col % 32 / 8)) * 8 +
+           col % 8;
+}
 
 // A register-streamed tile (k_pf_gemm_tile, k_pf_gemm_f32): a workgroup of 4
 // waves as 2 (rows) x 2 (columns); a wave owns 32 rows from m0 and NI weight-column subtiles
@@ -405,7 +440,13 @@ struct TileCtx {
                     if (MODE == GEMV_SILU) {
                         const float gv = acc[mi][ni][r] * rsa[r];
                         const float uv = acc[mi][ni + NO][r] * rsa[r];
-                        *p = (gv / (1.0f + expf(-gv))) * uv;
+                        const int e = hid_exp(a, row);
+                        const float t = ldexpf((gv / (1.0f + expf(-gv))) * uv, e);
+                        _Float16* o = hid_at(a, row, c[ni]);
+                        const _Float16 hi = (_Float16)t;
+                        o[0] = hi;
+                        o[512] = (_Float16)(t - (float)hi);
+                        if (c[ni] == 0) a.hid_rs[row] = ldexpf(1.0f, -e);
                     } else if (MODE == GEMV_STORE) {
                         const float v = acc[mi][ni][r] * rsa[r];
                         *p = bias[ni] ? v + bias[ni][c[ni]] : v;
@@ -892,6 +933,51 @@ __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a)
     }
     if (S > 0) scale_in(1, tp, tsp, dvp, mvp);
 
+    if constexpr (SILU && !SPLIT) {
+        // silu(gate) * up through LDS (this wave's 64 rows x 32 columns, one block of the next
+        // GEMM), then as its fragments: 16 bytes a lane, a fragment a store
+        constexpr int kLd = 36;  // 16-byte rows, 8 lanes of a read on distinct banks
+        float* hl = (float*)lds + wave * 64 * kLd;
+        __syncthreads();  // every wave is done with the stages
+        const int u0 = nt * 8 + wn * 2;
+        if (u0 >= a.n_sub) return;
+#pragma unroll
+        for (int mi = 0; mi < 4; ++mi) {
+            const int r0 = mt * kBigRows + (wm * 4 + mi) * 16 + 4 * (lane >> 4);
+            const float4 rsv = *(const float4*)(a.rs + r0);
+            const float rsa[4] = {rsv.x, rsv.y, rsv.z, rsv.w};
+#pragma unroll
+            for (int ni = 0; ni < 2; ++ni)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float gv = acc[mi][ni][r] * rsa[r], uv = acc[mi][ni + 2][r] * rsa[r];
+                    hl[(16 * mi + 4 * (lane >> 4) + r) * kLd + 16 * ni + l16] = (gv / (1.0f + expf(-gv))) * uv;
+                }
+        }
+        const int blk = a.hid_col0 / 32 + u0 / 2;
+        h8_t* out = (h8_t*)a.hid;
+#pragma unroll
+        for (int mi = 0; mi < 4; ++mi) {
+            const int tile = mt * 8 + wm * 4 + mi, row = 16 * tile + l16;
+            const int e = row < a.M ? hid_exp(a, row) : 0;
+            const float sc = ldexpf(1.0f, e);
+            const float* src = hl + (16 * mi + l16) * kLd + 8 * lc;
+            const float4 x0 = *(const float4*)src, x1 = *(const float4*)(src + 4);
+            const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+            h8_t hi, lo;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const float t = x[k] * sc;
+                hi[k] = (_Float16)t;
+                lo[k] = (_Float16)(t - (float)hi[k]);
+            }
+            h8_t* o = out + ((int64_t)tile * a.hid_nblk + blk) * 128 + lane;
+            o[0] = hi;
+            o[64] = lo;
+            if (u0 == 0 && lc == 0) a.hid_rs[row] = ldexpf(1.0f, -e);
+        }
+        return;
+    }
     // epilogue: lane holds rows 16 T + 4 (lane / 16) + r of weight column 16 q + l16
 #pragma unroll
     for (int mi = 0; mi < 4; ++mi) {
@@ -926,11 +1012,7 @@ __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a)
                 const int row = r0 + r;
                 if (row >= a.M) continue;
                 float* p = y + (int64_t)row * ldy + c;
-                if (SILU) {
-                    const float gv = acc[mi][ni][r] * rsa[r];
-                    const float uv = acc[mi][ni + 2][r] * rsa[r];
-                    *p = (gv / (1.0f + expf(-gv))) * uv;
-                } else if (MODE == GEMV_STORE) {
+                if (MODE == GEMV_STORE) {
                     const float v = acc[mi][ni][r] * rsa[r];
                     *p = bias ? v + bias[c] : v;
                 } else {
@@ -977,9 +1059,21 @@ __global__ __launch_bounds__(kBlock) void k_pf_reduce(const PfGemmArgs a) {
             w[2] += pv[k].z;
             w[3] += pv[k].w;
         }
-        float* y = a.seg[0].y + (int64_t)row * a.seg[0].ldy + col0;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) y[e] = (v[e] / (1.0f + expf(-v[e]))) * w[e];
+        for (int e = 0; e < 4; ++e) v[e] = (v[e] / (1.0f + expf(-v[e]))) * w[e];
+        const int ex = hid_exp(a, row);
+        const float sc = ldexpf(1.0f, ex);
+        h4_t hi, lo;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float t = v[e] * sc;
+            hi[e] = (_Float16)t;
+            lo[e] = (_Float16)(t - (float)hi[e]);
+        }
+        _Float16* o = hid_at(a, row, col0);
+        *(h4_t*)o = hi;
+        *(h4_t*)(o + 512) = lo;
+        if (col0 == 0) a.hid_rs[row] = ldexpf(1.0f, -ex);
         return;
     }
     // a 16-column subtile never straddles two segments, so neither do the 4 columns
@@ -1065,7 +1159,7 @@ __global__ __launch_bounds__(kBlock) void k_pf_reduce_rope(const PfGemmArgs a) {
 template <int KS, int NG>
 __global__ __launch_bounds__(kBlock) void k_pf_reduce_split(const PfGemmArgs a) {
     __shared__ double red_d[kWavesPerBlock];
-    __shared__ float red_f[kWavesPerBlock];
+    __shared__ float red_f[kWavesPerBlock], red_s[kWavesPerBlock];
     const int m = blockIdx.x, tid = threadIdx.x;
     const int K = a.n_sub * 16, ng = K / 8;
     if (m >= a.M) {
@@ -1104,7 +1198,8 @@ __global__ __launch_bounds__(kBlock) void k_pf_reduce_split(const PfGemmArgs a) 
                 for (int e = 0; e < 8; ++e) a.tap[8 * j + e] = v[i][e];
         }
     }
-    split_emit<NG, 4>(v, tid, m, K, a.split_w, a.split_eps, (h8_t*)a.split_xa, a.split_rs, red_d, red_f);
+    split_emit<NG, 4>(v, tid, m, K, a.split_w, a.split_eps, (h8_t*)a.split_xa, a.split_rs, a.split_xn, red_d, red_f,
+                      red_s);
 }
 
 
@@ -1117,7 +1212,7 @@ __global__ __launch_bounds__(kBlock) void k_pf_reduce_split(const PfGemmArgs a) 
 template <int KS, int NG>
 __global__ __launch_bounds__(kBlock) void k_pf_reduce_silu_split(const PfGemmArgs a) {
     __shared__ double red_d[kWavesPerBlock];
-    __shared__ float red_f[kWavesPerBlock];
+    __shared__ float red_f[kWavesPerBlock], red_s[kWavesPerBlock];
     const int m = blockIdx.x, tid = threadIdx.x;
     const int F = a.n_sub * 16, ng = F / 8;
     if (m >= a.M) {
@@ -1156,7 +1251,7 @@ __global__ __launch_bounds__(kBlock) void k_pf_reduce_silu_split(const PfGemmArg
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[i][e] = (g[e] / (1.0f + expf(-g[e]))) * u[e];
     }
-    split_emit<NG, 4>(v, tid, m, F, nullptr, 0.0f, (h8_t*)a.split_xa, a.split_rs, red_d, red_f);
+    split_emit<NG, 4>(v, tid, m, F, nullptr, 0.0f, (h8_t*)a.split_xa, a.split_rs, nullptr, red_d, red_f, red_s);
 }
 
 // ---------------------------------------------------------------- RoPE and KV store
@@ -1647,14 +1742,14 @@ bool pf_gemm_supported(int type, int64_t K, int64_t N) {
 }
 
 hipError_t launch_pf_split(const float* x, int64_t ldx, const float* norm_w, float eps, int K, int M, int Mpad,
-                           uint16_t* xa, float* rs, hipStream_t st) {
+                           uint16_t* xa, float* rs, hipStream_t st, float* xn) {
     if (K % 32 != 0 || K > kBlock * 8 * kSplitGroups || ldx % 4 != 0 || Mpad % kPfTileM != 0 || M > Mpad)
         return hipErrorInvalidValue;
     // a wave per row while a lane holds at most 20 groups (rows up to 10240), else a workgroup
     const int per1 = (K / 8 + 63) / 64;
 #define TF_SPLIT(NG, WPR, rows)                                                                              \
     hipLaunchKernelGGL((k_pf_split<NG, WPR>), dim3((unsigned)(Mpad / (rows))), dim3(kBlock), 0, st, x, ldx, \
-                       norm_w, eps, K, M, (h8_t*)xa, rs)
+                       norm_w, eps, K, M, (h8_t*)xa, rs, xn)
     if (per1 <= 2)
         TF_SPLIT(2, 1, kWavesPerBlock);
     else if (per1 <= 4)
@@ -1907,13 +2002,15 @@ hipError_t launch_pf_gemm(const PfGemmArgs& a, hipStream_t st, bool* fused) {
     const int t = a.seg[0].w.type;
     for (int s = 0; s < a.n_seg; ++s) {
         const PfSeg& g = a.seg[s];
-        if (!pf_gemm_supported(g.w.type, g.w.K, g.w.N) || g.w.type != t || g.w.K != a.K || !g.y)
+        if (!pf_gemm_supported(g.w.type, g.w.K, g.w.N) || g.w.type != t || g.w.K != a.K || (!g.y && a.mode != GEMV_SILU))
             return hipErrorInvalidValue;
         const int next = s + 1 < a.n_seg ? a.seg[s + 1].sub0 : a.n_sub;
         if (next - g.sub0 != g.w.N / 16) return hipErrorInvalidValue;
         if (a.mode == GEMV_SILU && (g.w2.type != t || g.w2.K != a.K || g.w2.N != g.w.N)) return hipErrorInvalidValue;
     }
     if (a.seg[0].sub0 != 0 || (a.mode == GEMV_SILU && a.n_seg != 1)) return hipErrorInvalidValue;
+    if (a.mode == GEMV_SILU && (!a.hid || !a.hid_rs || !a.xn || !a.wn_gate || !a.wn_up || a.hid_col0 % 32 != 0 || a.n_sub % 2 != 0))
+        return hipErrorInvalidValue;
     if (t == TF_HIP_TYPE_F32) {
         // register-streamed tiles only: 4 column subtiles per wave, 2 when that leaves
         // fewer than two workgroups per CU

@@ -92,6 +92,8 @@ struct tf_hip_ctx {
     int pf_state = -1;                 // -1 undecided, 0 per-token path, 1 matrix-core path ready
     int pf_cap = 0;                    // rows per prefill chunk (multiple of kPfTileM)
     float *px = nullptr, *pqkv = nullptr, *patt = nullptr, *ph = nullptr, *prs = nullptr;
+    float *phrs = nullptr, *pxn = nullptr;  // ph's row scales as an operand; sums of squares of the FFN's input rows
+    float* row_norms = nullptr;             // largest row norm of each layer's ffn_gate and ffn_up [layer][2]
     uint16_t* pxa = nullptr;            // activation fragments (hi, lo) of one chunk
     float* ppart = nullptr;             // split-K partial sums of the prefill GEMMs
     size_t ppart_floats = 0;
@@ -657,7 +659,8 @@ int ensure_pf(tf_hip_ctx* c) {
         const size_t kmax = std::max({D, F, (size_t)c->H});
         if ((rc = dalloc(c, &c->px, cap * D * 4)) || (rc = dalloc(c, &c->pqkv, cap * NQ * 4)) ||
             (rc = dalloc(c, &c->patt, cap * (size_t)c->H * 4)) || (rc = dalloc(c, &c->ph, cap * F * 4)) ||
-            (rc = dalloc(c, &c->prs, (size_t)cap * 4)) || (rc = dalloc(c, &c->pxa, cap * kmax * 2 * 2)))
+            (rc = dalloc(c, &c->prs, (size_t)cap * 4)) || (rc = dalloc(c, &c->pxa, cap * kmax * 2 * 2)) ||
+                (rc = dalloc(c, &c->phrs, (size_t)cap * 4)) || (rc = dalloc(c, &c->pxn, (size_t)cap * 4)))
             return rc;
         // up to 8 K slices of the widest non-SILU output (QKV or d_model)
         c->ppart_floats = 8 * (size_t)cap * std::max(NQ, D);
@@ -894,6 +897,7 @@ int prefill_mfma(tf_hip_ctx* c, int n) {
             a.split_eps = p.rms_eps;
         };
         bool x_split = false;  // the attention-norm split of px is in pxa already
+        bool h_split = false;  // the hidden rows' split is in pxa
         for (int l = 0; l < p.n_layer && e == hipSuccess; ++l) {
             auto M = [&](int k) { return TF_HIP_SLOT_LAYER(l, k); };
             auto V = [&](int k) { return vec(c, TF_HIP_SLOT_LAYER(l, k)); };
@@ -951,11 +955,12 @@ int prefill_mfma(tf_hip_ctx* c, int n) {
                 a.mode = GEMV_RESID;
                 seg(a, M(TF_HIP_LAYER_O), c->px, D, nullptr);
                 fuse_split(a, V(TF_HIP_LAYER_FFN_NORM));
+                a.split_xn = c->pxn;
                 bool done = false;
                 chk(launch_pf_gemm(a, c->st, &done));
                 if (!done)
                     chk(launch_pf_split(c->px, D, V(TF_HIP_LAYER_FFN_NORM), p.rms_eps, D, nc, Mpad, c->pxa,
-                                        c->prs, c->st));
+                                        c->prs, c->st, c->pxn));
             }
             {
                 // gate/up's large tiles (128 output columns) past whole rounds over the CUs: the
@@ -975,28 +980,34 @@ int prefill_mfma(tf_hip_ctx* c, int n) {
                     PfSeg& sg = a.seg[a.n_seg++];
                     sg.w = devmat_rows(mat(c, M(TF_HIP_LAYER_GATE)), c0, c1 - c0);
                     sg.w2 = devmat_rows(mat(c, M(TF_HIP_LAYER_UP)), c0, c1 - c0);
-                    sg.y = c->ph + c0;
-                    sg.ldy = F;
-                    sg.bias = nullptr;
-                    sg.sub0 = 0;
                     a.n_sub = (c1 - c0) / 16;
+                    a.hid = (uint16_t*)c->ph;  // 4 bytes an element either way
+                    a.hid_rs = c->phrs;
+                    a.hid_col0 = c0;
+                    a.hid_nblk = F / 32;
+                    a.xn = c->pxn;
+                    a.wn_gate = c->row_norms + 2 * l;
+                    a.wn_up = c->row_norms + 2 * l + 1;
                     if (fuse) {  // a K-split reduce also splits the hidden rows
                         a.split_xa = c->pxa;
                         a.split_rs = c->prs;
                     }
                     chk(launch_pf_gemm(a, c->st, done));
                 };
-                bool done = false;
+                h_split = false;
                 if (ncA > 0 && ncA < ncol) {
                     gateup(0, ncA * 128, false, nullptr);
                     gateup(ncA * 128, F, false, nullptr);
                 } else {
-                    gateup(0, F, true, &done);
+                    gateup(0, F, true, &h_split);
                 }
-                if (!done) chk(launch_pf_split(c->ph, F, nullptr, 0.0f, F, nc, Mpad, c->pxa, c->prs, c->st));
             }
             {
                 PfGemmArgs a = base(F);
+                if (!h_split) {  // the hidden rows came out as an operand in ph
+                    a.xa = (const uint16_t*)c->ph;
+                    a.rs = c->phrs;
+                }
                 a.mode = GEMV_RESID;
                 seg(a, M(TF_HIP_LAYER_DOWN), c->px, D, nullptr);
                 if (last) {
@@ -1090,6 +1101,7 @@ int tf_hip_create(int device, const tf_hip_hparams* hp, tf_hip_ctx** out) {
         (rc = dalloc(c, &c->part_ml, (size_t)p.n_head * S * 2 * 4)) ||
         (rc = dalloc(c, &c->ctl, sizeof(Ctl))) ||
         (rc = dalloc(c, &c->hist, (size_t)p.max_seq * 4)) ||
+        (rc = dalloc(c, &c->row_norms, (size_t)p.n_layer * 2 * 4)) ||
         (rc = dalloc(c, &c->rope_cos, (size_t)p.max_seq * (p.head_dim / 2) * 4)) ||
         (rc = dalloc(c, &c->rope_sin, (size_t)p.max_seq * (p.head_dim / 2) * 4)))
         return bail(rc);
@@ -1098,7 +1110,8 @@ int tf_hip_create(int device, const tf_hip_hparams* hp, tf_hip_ctx** out) {
     std::memset(c->ctl_host, 0, sizeof(Ctl));
     if (hipMemset(c->ctl, 0, sizeof(Ctl)) != hipSuccess || hipMemset(c->kc, 0, c->kv_layer * p.n_layer * 4) != hipSuccess ||
         hipMemset(c->vc, 0, c->kv_layer * p.n_layer * 4) != hipSuccess ||
-        hipMemset(c->taps, 0, (size_t)(p.n_layer + 1) * D * 4) != hipSuccess)
+        hipMemset(c->taps, 0, (size_t)(p.n_layer + 1) * D * 4) != hipSuccess ||
+        hipMemset(c->row_norms, 0, (size_t)p.n_layer * 2 * 4) != hipSuccess)
         return bail(TF_HIP_EDEVICE);
     if (hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess) return bail(TF_HIP_EDEVICE);
     if (const char* lg = std::getenv("TF_HIP_LOG"); lg && *lg && std::strcmp(lg, "0") != 0)
@@ -1198,6 +1211,11 @@ int tf_hip_upload_tensor(tf_hip_ctx* c, int slot, int t, int64_t ne0, int64_t ne
     DevMat m;
     std::vector<void*> owned;
     if (e == hipSuccess) e = make_devmat(t, K, N, raw, m, owned, c->st);
+    if (e == hipSuccess && (kind == TF_HIP_LAYER_GATE || kind == TF_HIP_LAYER_UP)) {
+        float* norm = c->row_norms + 2 * ((slot - 16) / TF_HIP_LAYER_COUNT) + (kind == TF_HIP_LAYER_UP);
+        if (c->mats[(size_t)slot].valid()) e = hipMemsetAsync(norm, 0, sizeof(float), c->st);  // uploaded before
+        if (e == hipSuccess) e = launch_row_norm_max(m, norm, c->st);
+    }
     if (e == hipSuccess) e = hipStreamSynchronize(c->st);
     (void)hipFree(raw);
     if (e != hipSuccess) {

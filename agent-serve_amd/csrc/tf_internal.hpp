@@ -197,6 +197,15 @@ struct PfGemmArgs {
     float* split_rs = nullptr;
     const float* split_w = nullptr;
     float split_eps = 0.0f;
+    float* split_xn = nullptr;     // GEMV_RESID: the split rows' sums of squares, when wanted
+    // GEMV_SILU: the silu * up rows go out as the next GEMM's operand (hid, its row scales hid_rs),
+    // columns from hid_col0 on of hid_nblk blocks a row; scaled by a bound from the input rows' sums
+    // of squares xn and the largest norms of a gate and of an up row (launch_row_norm_max). A
+    // K-split reduce with split_xa set splits them there by their largest value instead.
+    uint16_t* hid = nullptr;
+    float* hid_rs = nullptr;
+    int hid_col0 = 0, hid_nblk = 0;
+    const float *xn = nullptr, *wn_gate = nullptr, *wn_up = nullptr;
     // GEMV_STORE of the q, k and v segments, rope_cos set: launch_pf_rope_store of the rows
     // (q rotated into its segment's rows, k rotated and v into the cache at pos0 + row)
     const float* rope_cos = nullptr;
@@ -253,7 +262,7 @@ hipError_t launch_pf_small_attn(const PfSmallAttn& a, int hd, hipStream_t st);
 bool pf_gemm_supported(int type, int64_t K, int64_t N);
 // xa needs Mpad * K * 2 halves, rs Mpad floats.
 hipError_t launch_pf_split(const float* x, int64_t ldx, const float* norm_w, float eps, int K, int M, int Mpad,
-                           uint16_t* xa, float* rs, hipStream_t st);
+                           uint16_t* xa, float* rs, hipStream_t st, float* xn = nullptr);
 hipError_t launch_pf_gemm(const PfGemmArgs& a, hipStream_t st, bool* fused = nullptr);
 hipError_t launch_embed_rows(const DevMat& emb, const int32_t* tok, int n, float* x, int D, hipStream_t st);
 hipError_t launch_pf_rope_store(float* qkv, int64_t ld, int n, int H, int G, int hd, const float* rope_cos,
@@ -309,6 +318,8 @@ size_t gemv_lds_bytes(int64_t K);
 hipError_t launch_attn_decode(const AttnArgs& a, hipStream_t st);
 hipError_t launch_embed(const DevMat& emb, float* x, Ctl* ctl, int32_t* hist, int D, hipStream_t st);
 hipError_t launch_dequant_rows(const DevMat& m, int64_t row0, int64_t nrows, float* out, hipStream_t st);
+// The largest 2-norm of a row of m, rounded up, into *out (where it is larger).
+hipError_t launch_row_norm_max(const DevMat& m, float* out, hipStream_t st);
 hipError_t launch_repack(int type, const uint8_t* raw, int64_t K, int64_t N, DevMat& m, hipStream_t st);
 hipError_t launch_rmsnorm_rows(const float* x, const float* w, int n, int rows, float eps, float* out,
                                hipStream_t st);
