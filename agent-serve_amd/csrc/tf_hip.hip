@@ -91,8 +91,10 @@ struct tf_hip_ctx {
     int pf_opt = TF_HIP_PREFILL_MFMA;  // requested prefill path
     int pf_state = -1;                 // -1 undecided, 0 per-token path, 1 matrix-core path ready
     int pf_cap = 0;                    // rows per prefill chunk (multiple of kPfTileM)
-    float *px = nullptr, *pqkv = nullptr, *patt = nullptr, *ph = nullptr, *prs = nullptr;
+    float *px = nullptr, *pqkv = nullptr, *ph = nullptr, *prs = nullptr;
     float *phrs = nullptr, *pxn = nullptr;  // ph's row scales as an operand; sums of squares of the FFN's input rows
+    float* pvmax = nullptr;                 // largest value element of an attention call: two words, used in turn
+    int pvmax_i = 0;                        // the word that is 0 now
     float* row_norms = nullptr;             // largest row norm of each layer's ffn_gate and ffn_up [layer][2]
     uint16_t* pxa = nullptr;            // activation fragments (hi, lo) of one chunk
     float* ppart = nullptr;             // split-K partial sums of the prefill GEMMs
@@ -658,9 +660,9 @@ int ensure_pf(tf_hip_ctx* c) {
         const size_t D = (size_t)p.n_embd, F = (size_t)p.n_ff, NQ = (size_t)c->H + 2 * (size_t)c->KVd;
         const size_t kmax = std::max({D, F, (size_t)c->H});
         if ((rc = dalloc(c, &c->px, cap * D * 4)) || (rc = dalloc(c, &c->pqkv, cap * NQ * 4)) ||
-            (rc = dalloc(c, &c->patt, cap * (size_t)c->H * 4)) || (rc = dalloc(c, &c->ph, cap * F * 4)) ||
-            (rc = dalloc(c, &c->prs, (size_t)cap * 4)) || (rc = dalloc(c, &c->pxa, cap * kmax * 2 * 2)) ||
-                (rc = dalloc(c, &c->phrs, (size_t)cap * 4)) || (rc = dalloc(c, &c->pxn, (size_t)cap * 4)))
+            (rc = dalloc(c, &c->ph, cap * F * 4)) || (rc = dalloc(c, &c->prs, (size_t)cap * 4)) ||
+            (rc = dalloc(c, &c->pxa, cap * kmax * 2 * 2)) || (rc = dalloc(c, &c->pvmax, 2 * sizeof(float))) ||
+            (rc = dalloc(c, &c->phrs, (size_t)cap * 4)) || (rc = dalloc(c, &c->pxn, (size_t)cap * 4)))
             return rc;
         // up to 8 K slices of the widest non-SILU output (QKV or d_model)
         c->ppart_floats = 8 * (size_t)cap * std::max(NQ, D);
@@ -668,6 +670,7 @@ int ensure_pf(tf_hip_ctx* c) {
         const size_t count_bytes = D / 16 * sizeof(int);
         if ((rc = dalloc(c, &c->pf_count, count_bytes))) return rc;
         HIPCHK(c, hipMemset(c->pf_count, 0, count_bytes));
+        HIPCHK(c, hipMemset(c->pvmax, 0, 2 * sizeof(float)));
         // attention of a chunk covers at most max_seq positions
         c->pattn_ws_bytes = pf_attn_ws_bytes(p.head_dim, p.n_kv_head, p.max_seq);
         if ((rc = dalloc(c, &c->pattn_ws, c->pattn_ws_bytes))) return rc;
@@ -947,9 +950,10 @@ int prefill_mfma(tf_hip_ctx* c, int n) {
                 if (last) chk(prefill_last_row(c, l, c->pqkv + (int64_t)(nc - 1) * NQ, nc, start + n - 1, start));
                 continue;
             }
+            const PfAttnOperand op{c->pxa, c->prs, c->pvmax + c->pvmax_i, c->pvmax + (c->pvmax_i ^ 1)};
+            c->pvmax_i ^= 1;
             chk(launch_pf_attn(c->pqkv, NQ, kc, vc, p.kv_layout, p.n_head, p.n_kv_head, p.head_dim, p.max_seq, nc,
-                               pos0, start, c->patt, Hd, c->pattn_ws, c->pattn_ws_bytes, c->st));
-            chk(launch_pf_split(c->patt, Hd, nullptr, 0.0f, Hd, nc, Mpad, c->pxa, c->prs, c->st));
+                               pos0, start, nullptr, 0, c->pattn_ws, c->pattn_ws_bytes, c->st, op));
             {
                 PfGemmArgs a = base(Hd);
                 a.mode = GEMV_RESID;

@@ -269,12 +269,20 @@ hipError_t launch_pf_rope_store(float* qkv, int64_t ld, int n, int H, int G, int
                                 const float* rope_sin, int pos0, float* kc, float* vc, int layout, int max_seq,
                                 hipStream_t st);
 bool pf_attn_supported(int hd, int n_rep);
+// Where launch_pf_attn writes its rows as the next GEMM's operand (xa, row scales rs) instead of
+// as floats: vmax is 0 before the launch and takes the largest value element; vmax_next is set to 0
+// for the launch after.
+struct PfAttnOperand {
+    uint16_t* xa = nullptr;
+    float* rs = nullptr;
+    float *vmax = nullptr, *vmax_next = nullptr;
+};
 // Workspace of launch_pf_attn for attention over n_keys positions: the packed key/value
 // tile records.
 size_t pf_attn_ws_bytes(int hd, int G, int n_keys);
 hipError_t launch_pf_attn(const float* q, int64_t ldq, const float* kc, const float* vc, int layout, int H, int G,
                           int hd, int max_seq, int n, int pos0, int att_start, float* out, int64_t ldo, void* ws,
-                          size_t ws_bytes, hipStream_t st);
+                          size_t ws_bytes, hipStream_t st, const PfAttnOperand& op = {});
 hipError_t launch_pf_tail(Ctl* ctl, int pos_last, const int32_t* hist, const float* xrow, float* x, int D,
                           hipStream_t st);
 
