@@ -28,6 +28,8 @@
 // both far inside the 1e-3 parity bound. Scaling rows by 2^e (max |x| in [2^14, 2^15))
 // keeps hi and lo in fp16 range and off its subnormals; the epilogue multiplies the
 // exact inverse back.
+#include <type_traits>
+
 #include "dev_common.hpp"
 #include "tf_internal.hpp"
 
@@ -334,21 +336,54 @@ __global__ __launch_bounds__(kBlock) void k_pf_split(const float* x, int64_t ldx
 // Field of the segment holding output subtile u (uniform per wave: scalar selects).
 #define PF_SEL(s, f) ((s) == 0 ? a.seg[0].f : ((s) == 1 ? a.seg[1].f : a.seg[2].f))
 
-// Hidden rows as the next GEMM's operand: h = silu(g) u with |g| and |u| at most the
-// row's norm times the largest norm of a gate / up row, so |h| < 2^hid_exp without a pass over the
-// row, which no workgroup has whole. The operand's power of two comes from that bound instead
-// of the row's largest value: fp16's pair then keeps 22 bits of every value down to 2^-18 of the
-// bound, and 2^-40 of the bound below that. The bound is 2^7 to 2^9 above the row's largest value
-// for N(0, sigma) weights; one 2^14 above would still leave errors at 2^-26 of it. (Written as fp32
-// rows and split in a pass of their own, 11.7 us a layer at 512 rows of 8,192: a whole 512-token
-// prompt of the Llama-3.2-1B shape 4.10 -> 3.87 ms, 2,900 tokens of the Qwen2.5-1.5B shape 29.6 ->
-// 27.9, 333 on 4-bit weights 3.75 -> 3.54.)
+// An operand whose rows no workgroup has whole (the hidden rows): the row scale is 2^-e for an e
+// that a bound gives, and each 32-element block has an exponent kx of its own, so that how loose the bound is costs no bits. A block whose largest value m gives 2^4 <= m 2^e < 2^15 is
+// written as v 2^e (kx 0): fp16's pair hi + lo keeps 22 bits of what is at least 2^-7 of m, and the
+// rest to 2^-29 of m. Any other block is written as v 2^(e + kx), m 2^(e + kx) in [2^14, 2^15). The GEMM
+// takes 2^kx out of the block's sum, an exact operation, in a loop of its own that runs where a flag
+// says that one of 128 rows has such a block: 317 us for 252 at 2,900 rows of 8,960, as much as the pass
+// over fp32 rows that a scale from the row's largest value takes (a whole prompt with one gate and one up
+// row 2^8 times the others: 2,900 tokens of the Qwen2.5-1.5B shape 27.2 -> 28.8 ms, 512 of the
+// Llama-3.2-1B shape 3.77 -> 3.93). (One loop with a branch per block in it: every prompt 2 to 6 %, and in
+// Q6_K, whose registers then spill, 1.8 times the time.)
+// (kx and e + kx stay in -126 .. 126, where their powers of two are floats.)
+__device__ __forceinline__ int blk_exp(float amax, int e) {
+    int x;
+    (void)frexpf(amax, &x);  // amax in [2^(x - 1), 2^x)
+    x += e;
+    if (!(amax > 0.0f) || !(amax < INFINITY) || (x >= 5 && x <= 15)) return 0;
+    const int hi = 126 - e < 126 ? 126 - e : 126;
+    return 15 - x < hi ? (15 - x > -126 ? 15 - x : -126) : hi;
+}
+// The largest of the lanes l16 + 0, 16, 32 and 48, in each of them.
+__device__ __forceinline__ float max_of_4(float m) {
+    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+    m = fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+    const auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+    return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
+}
+// The largest of an aligned eight lanes, in each of them.
+__device__ __forceinline__ float max_of_8(float m) {
+    m = fmaxf(m, dpp<kDppXor1>(m));
+    m = fmaxf(m, dpp<kDppXor2>(m));
+    return fmaxf(m, dpp<kDppHalfMirror>(m));
+}
+// 2^-kx for byte r of the exponents of four rows.
+__device__ __forceinline__ float blk_unscale(uint32_t kx, int r) {
+    return __uint_as_float((uint32_t)(127 - (int)(int8_t)(kx >> (8 * r))) << 23);
+}
+// e of the hidden row: h = silu(g) u, |g| and |u| at most the input row's norm times the largest norm
+// of a gate / up row, so |h| < 2^(21 - e). For N(0, sigma) weights that bound is 2^6 to 2^15 above
+// the blocks' largest values, inside the range that needs no exponent. (Written as fp32 rows
+// and split in a pass of their own, 11.7 us a layer at 512 rows of 8,192: a whole 512-token prompt of
+// the Llama-3.2-1B shape 4.10 -> 3.87 ms, 2,900 tokens of the Qwen2.5-1.5B shape 29.6 -> 27.9, 333 on
+// 4-bit weights 3.75 -> 3.54.)
 __device__ __forceinline__ int hid_exp(const PfGemmArgs& a, int row) {
     int ex, eg, eu;
     (void)frexpf(a.xn[row], &ex);
     (void)frexpf(*a.wn_gate, &eg);
     (void)frexpf(*a.wn_up, &eu);
-    const int e = 15 - (ex + eg + eu);
+    const int e = 21 - (ex + eg + eu);
     return e < -100 ? -100 : (e > 100 ? 100 : e);
 }
 // Element (row, col) of the operand: its hi half; the lo half 512 halves on.
@@ -356,6 +391,16 @@ __device__ __forceinline__ _Float16* hid_at(const PfGemmArgs& a, int row, int co
     col += a.hid_col0;
     return (_Float16*)a.hid + (((int64_t)(row / 16) * a.hid_nblk + col / 32) * 128 + row % 16 + 16 * (col % 32 / 8)) * 8 +
            col % 8;
+}
+
+// The exponent of the block that holds column col.
+__device__ __forceinline__ int8_t* hid_kx_at(const PfGemmArgs& a, int row, int col) {
+    return a.hid_kx + (int64_t)((col + a.hid_col0) / 32) * a.Mpad + row;
+}
+// Whether one of the 128 rows around row has a block exponent (a scalar load: row is the wave's).
+__device__ __forceinline__ bool has_exps(const PfGemmArgs& a, int row) {
+    typedef const __attribute__((address_space(4))) uint32_t* cptr;
+    return a.kxf && *(cptr)(uintptr_t)(a.kxf + __builtin_amdgcn_readfirstlane(row / 128)) != 0;
 }
 
 // A register-streamed tile (k_pf_gemm_tile, k_pf_gemm_f32): a workgroup of 4
@@ -421,9 +466,74 @@ struct TileCtx {
         for (int mi = 0; mi < MI; ++mi)
             ap[mi] = (const TF_GLOBAL h8_t*)a.xa + (int64_t)(m0 / 16 + mi) * nblk * 128 + lane;
     }
+    // GEMV_SILU: silu(gate) * up as the next GEMM's operand. A block is two column subtiles: both this
+    // wave's (NO 2), or one of this wave's and one of its neighbour's along the columns, the two
+    // largest values exchanged through LDS. Every wave of the workgroup comes here.
+    __device__ __forceinline__ void epilogue_hidden(const PfGemmArgs& a, const f4_t (&acc)[MI][NI]) const {
+        __shared__ float mx[4][16 * MI];
+        const int wave = threadIdx.x >> 6;
+        float h[MI][4][NO], m[MI][4];
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi) {
+            const float4 rsv = *(const float4*)(a.rs + m0 + 16 * mi + 4 * lc);
+            const float rsa[4] = {rsv.x, rsv.y, rsv.z, rsv.w};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                m[mi][r] = 0.0f;
+#pragma unroll
+                for (int ni = 0; ni < NO; ++ni) {
+                    const float gv = acc[mi][ni][r] * rsa[r];
+                    const float uv = acc[mi][ni + NI - NO][r] * rsa[r];
+                    h[mi][r][ni] = (gv / (1.0f + expf(-gv))) * uv;
+                    m[mi][r] = fmaxf(m[mi][r], fabsf(h[mi][r][ni]));
+                }
+                m[mi][r] = max_of_8(m[mi][r]);
+                m[mi][r] = fmaxf(m[mi][r], dpp<kDppMirror>(m[mi][r]));
+            }
+        }
+        if (NO == 1) {
+#pragma unroll
+            for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (l16 == 0) mx[wave][16 * mi + 4 * lc + r] = m[mi][r];
+            __syncthreads();
+            const int other = WM == 2 ? wave ^ 2 : wave ^ 1;
+#pragma unroll
+            for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) m[mi][r] = fmaxf(m[mi][r], mx[other][16 * mi + 4 * lc + r]);
+        }
+        bool any = false;
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = m0 + 16 * mi + 4 * lc + r;
+                if (row >= a.M || !ok[0]) continue;  // n_sub is even: the block's two subtiles are both there
+                const int e = hid_exp(a, row), k = blk_exp(m[mi][r], e);
+                const float sc = ldexpf(1.0f, e + k);
+#pragma unroll
+                for (int ni = 0; ni < NO; ++ni) {
+                    const float t = h[mi][r][ni] * sc;
+                    _Float16* o = hid_at(a, row, c[ni]);
+                    const _Float16 hi = (_Float16)t;
+                    o[0] = hi;
+                    o[512] = (_Float16)(t - (float)hi);
+                }
+                if (c[0] % 32 == 0) *hid_kx_at(a, row, c[0]) = (int8_t)k;
+                if (c[0] == 0) a.hid_rs[row] = ldexpf(1.0f, -e);
+                any |= k != 0;
+            }
+        if (__builtin_amdgcn_ballot_w64(any) != 0 && lane == 0) a.hid_kxf[m0 / 128] = 1;
+    }
     // lane holds rows m0 + 16 mi + 4 (lane / 16) + r of output column c[ni], scaled back by
     // the row scales: store (+ bias), residual add (+ the tap row) or silu(gate) * up
     __device__ __forceinline__ void epilogue(const PfGemmArgs& a, const f4_t (&acc)[MI][NI]) const {
+        if constexpr (MODE == GEMV_SILU) {
+            epilogue_hidden(a, acc);
+            return;
+        }
 #pragma unroll
         for (int mi = 0; mi < MI; ++mi) {
             const int r0 = m0 + 16 * mi + 4 * (lane >> 4);
@@ -437,17 +547,7 @@ struct TileCtx {
                 for (int ni = 0; ni < NO; ++ni) {
                     if (!ok[ni]) continue;
                     float* p = y[ni] + (int64_t)row * ldy[ni] + c[ni];
-                    if (MODE == GEMV_SILU) {
-                        const float gv = acc[mi][ni][r] * rsa[r];
-                        const float uv = acc[mi][ni + NO][r] * rsa[r];
-                        const int e = hid_exp(a, row);
-                        const float t = ldexpf((gv / (1.0f + expf(-gv))) * uv, e);
-                        _Float16* o = hid_at(a, row, c[ni]);
-                        const _Float16 hi = (_Float16)t;
-                        o[0] = hi;
-                        o[512] = (_Float16)(t - (float)hi);
-                        if (c[ni] == 0) a.hid_rs[row] = ldexpf(1.0f, -e);
-                    } else if (MODE == GEMV_STORE) {
+                    if (MODE == GEMV_STORE) {
                         const float v = acc[mi][ni][r] * rsa[r];
                         *p = bias[ni] ? v + bias[ni][c[ni]] : v;
                     } else {
@@ -524,10 +624,11 @@ __global__ __launch_bounds__(256) void k_pf_gemm_tile(const PfGemmArgs a) {
         typename W::Raw bw[NI][2];  // [column subtile][block]: the lane's weight bytes
         uint32_t d[NI][SW];         // the scale words of the stage's two blocks
         uint16_t d2[NI];            // Q6_K: d of the stage's blocks
+        uint32_t kx[MI][2];         // the lane's four rows' block exponents
     };
     const int S = SPLIT ? K / 64 / a.ks : K / 64;  // stages (two blocks) of this K slice
     const int sb = SPLIT ? t.kslice * S : 0;       // its first stage
-    auto load = [&](int s, Stage& g) {
+    auto load = [&](auto has_exp, int s, Stage& g) {
         s = sb + (s < S ? s : S - 1);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -536,6 +637,9 @@ __global__ __launch_bounds__(256) void k_pf_gemm_tile(const PfGemmArgs a) {
             for (int mi = 0; mi < MI; ++mi) {
                 g.ah[mi][j] = ap[mi][blk * 128];
                 g.al[mi][j] = ap[mi][blk * 128 + 64];
+                if (decltype(has_exp)::value)
+                    g.kx[mi][j] = *(const TF_GLOBAL uint32_t*)((const TF_GLOBAL uint8_t*)a.kx + (int64_t)blk * a.Mpad +
+                                                               t.m0 + 16 * mi + 4 * t.lc);
             }
 #pragma unroll
             for (int ni = 0; ni < NI; ++ni) {
@@ -555,7 +659,8 @@ __global__ __launch_bounds__(256) void k_pf_gemm_tile(const PfGemmArgs a) {
                 for (int w = 0; w < SW; ++w) g.d[ni][w] = sp[ni][SW * s + w];
     };
     const h8_t ones = {1, 1, 1, 1, 1, 1, 1, 1};
-    auto compute = [&](const Stage& g) {
+    auto compute = [&](auto has_exp, const Stage& g) {
+        constexpr bool EXP = decltype(has_exp)::value;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             h8_t bh[NI], bl[NI];
@@ -590,6 +695,16 @@ __global__ __launch_bounds__(256) void k_pf_gemm_tile(const PfGemmArgs a) {
 #pragma unroll
                     for (int ni = 0; ni < NI; ++ni)
                         tb[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_f16(g.ah[mi][j], bl[ni], tb[mi][ni], 0, 0, 0);
+            if (EXP)
+#pragma unroll
+                for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float f = blk_unscale(g.kx[mi][j], r);
+#pragma unroll
+                        for (int ni = 0; ni < NI; ++ni) tb[mi][ni][r] *= f;
+                        if (W::kMin) ts[mi][r] *= f;
+                    }
 #pragma unroll
             for (int ni = 0; ni < NI; ++ni) {
                 float dv, mv = 0.0f;
@@ -606,16 +721,22 @@ __global__ __launch_bounds__(256) void k_pf_gemm_tile(const PfGemmArgs a) {
             }
         }
     };
-    Stage s0, s1;
-    load(0, s0);
-    int s = 0;
-    for (; s + 2 <= S; s += 2) {
-        load(s + 1, s1);
-        compute(s0);
-        load(s + 2, s0);
-        compute(s1);
-    }
-    if (s < S) compute(s0);
+    auto run = [&](auto has_exp) {
+        Stage s0, s1;
+        load(has_exp, 0, s0);
+        int s = 0;
+        for (; s + 2 <= S; s += 2) {
+            load(has_exp, s + 1, s1);
+            compute(has_exp, s0);
+            load(has_exp, s + 2, s0);
+            compute(has_exp, s1);
+        }
+        if (s < S) compute(has_exp, s0);
+    };
+    if (MODE == GEMV_RESID && has_exps(a, t.m0))
+        run(std::true_type{});
+    else
+        run(std::false_type{});
     if (SPLIT)
         t.epilogue_part(a, acc);
     else
@@ -626,7 +747,8 @@ __global__ __launch_bounds__(256) void k_pf_gemm_tile(const PfGemmArgs a) {
 // fragments (their sum, exact in fp32, is the row's 22-bit value); the weights are loaded as
 // they lie. Within a 32-element block, MFMA j (0..7) takes from lane l the element
 // k = 8 (l / 16) + j: the 8 consecutive values each lane holds of both operands, a
-// reordering of the block's terms. No block scales: every MFMA accumulates into acc.
+// reordering of the block's terms. No block scales: every MFMA accumulates into acc (GEMV_RESID: the
+// operand's block exponents are taken out of x).
 template <int MODE, int NI>
 __global__ __launch_bounds__(256) void k_pf_gemm_f32(const PfGemmArgs a) {
     const TileCtx<MODE, NI> t(a);
@@ -648,6 +770,11 @@ __global__ __launch_bounds__(256) void k_pf_gemm_f32(const PfGemmArgs a) {
             const h8_t hi = ap[mi][blk * 128], lo = ap[mi][blk * 128 + 64];
 #pragma unroll
             for (int j = 0; j < 8; ++j) x[mi][j] = (float)hi[j] + (float)lo[j];
+            if (MODE == GEMV_RESID && a.kx) {
+                const int k = a.kx[(int64_t)blk * a.Mpad + t.m0 + 16 * mi + t.l16];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) x[mi][j] = ldexpf(x[mi][j], -k);
+            }
         }
         float w[NI][8];
 #pragma unroll
@@ -687,7 +814,10 @@ constexpr int kBigStages = 4;          // LDS buffers: one in use, three loading
 // A stage's weight bytes: 256 rows x 64 at most (F16); Q6_K's two streams, lo then hi, in 8 KiB
 constexpr int big_b_bytes(int type) { return type == TF_HIP_TYPE_Q6_K ? 8 * 1024 : 16 * 1024; }
 constexpr int kBigHiOff = 4 * 1024;
-constexpr int big_stage_bytes(int type) { return kBigABytes + big_b_bytes(type) + 1024; }  // + a scale word per weight row
+// + for each of the 8 waves that load them, the scale words of 32 weight rows and the block exponents of
+// 16 activation rows
+constexpr int kBigScaleBytes = 128 + 16;
+constexpr int big_stage_bytes(int type) { return kBigABytes + big_b_bytes(type) + 8 * kBigScaleBytes; }
 // Beside the stages, Q6_K keeps d (fp16) of the workgroup's 256 weight rows for the
 // super-blocks of 8 blocks that a slice of S blocks can touch: [super-block][row].
 constexpr size_t big_lds_bytes(int type, int S) {
@@ -780,7 +910,14 @@ __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a)
         dsrc = (const TF_GLOBAL uint32_t*)(ws + (int64_t)c * nblk * W::kScale);
     }
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds;
-    auto issue = [&](int s) {  // stage s into buffer s % 4: 4 loads per wave
+    // lanes 32..35 (with scales; 0..3 without): the block exponents of rows 16 wave + 4 (lane % 4) ..
+    const TF_GLOBAL uint8_t* ksrc = (const TF_GLOBAL uint8_t*)a.kx + mt * kBigRows + 16 * wave + 4 * (lane & 3);
+    auto issue_exps = [&](int s) {
+        const uint32_t m0 = __builtin_amdgcn_readfirstlane(
+            lds0 + (uint32_t)((s % kBigStages) * kBigStageBytes + kBigABytes + kBigBBytes + kBigScaleBytes * wave + 128));
+        if (lane < 4) lds_dma4(ksrc + (int64_t)(s0 + s) * a.Mpad, m0);
+    };
+    auto issue = [&](auto has_exp, int s) {  // stage s into buffer s % 4: kLoads loads per wave
         const int blk = s0 + s;
         const uint32_t base = lds0 + (uint32_t)((s % kBigStages) * kBigStageBytes);
 #pragma unroll
@@ -802,8 +939,17 @@ __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a)
                 lds_dma16(bsrc[j] + (int64_t)blk * W::kBytes, __builtin_amdgcn_readfirstlane(bb + 1024u * (2 * wave + j)));
         }
         if (W::kScale) {
-            const uint32_t m0 = __builtin_amdgcn_readfirstlane(base + (uint32_t)(kBigABytes + kBigBBytes + 128 * wave));
-            if (lane < 32) lds_dma4(dsrc + (W::kScale == 2 ? blk / 2 : blk), m0);
+            const uint32_t m0 =
+                __builtin_amdgcn_readfirstlane(base + (uint32_t)(kBigABytes + kBigBBytes + kBigScaleBytes * wave));
+            const TF_GLOBAL uint32_t* d = dsrc + (W::kScale == 2 ? blk / 2 : blk);
+            if (decltype(has_exp)::value) {
+                if (lane >= 32) d = (const TF_GLOBAL uint32_t*)(ksrc + (int64_t)blk * a.Mpad);
+                if (lane < 36) lds_dma4(d, m0);
+            } else {
+                if (lane < 32) lds_dma4(d, m0);
+            }
+        } else if (decltype(has_exp)::value) {
+            issue_exps(s);
         }
     };
     constexpr int kLoads = 2 + NB + (W::kScale ? 1 : 0) + (W::kPair ? 1 : 0);
@@ -824,9 +970,12 @@ __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a)
     }
 
     const int wm = wave & 1, wn = wave >> 1;
-    int qb[4];  // this wave's weight-column subtiles
+    int qb[4], sq[4];  // this wave's weight-column subtiles; their columns' scale words
 #pragma unroll
-    for (int ni = 0; ni < 4; ++ni) qb[ni] = SILU ? (ni < 2 ? wn * 2 + ni : 8 + wn * 2 + ni - 2) : wn * 4 + ni;
+    for (int ni = 0; ni < 4; ++ni) {
+        qb[ni] = SILU ? (ni < 2 ? wn * 2 + ni : 8 + wn * 2 + ni - 2) : wn * 4 + ni;
+        sq[ni] = qb[ni] / 2 * (kBigScaleBytes / 4) + qb[ni] % 2 * 16 + l16;
+    }
 
     f4_t acc[4][4];
 #pragma unroll
@@ -840,21 +989,27 @@ __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a)
     f4_t tp[2][4];  // pending block sums: rows half 1 of the previous block
     f4_t tsp[2];    // Q4_1: their rows' block sums
     float dvp[4], mvp[4];
-    auto scale_in = [&](int half, const f4_t (&t)[2][4], const f4_t (&ts)[2], const float (&dv)[4],
-                        const float (&mv)[4]) {
+    uint32_t kxp[2];  // block exponents of their rows
+    auto scale_in = [&](auto has_exp, int half, const f4_t (&t)[2][4], const f4_t (&ts)[2], const float (&dv)[4],
+                        const float (&mv)[4], const uint32_t (&kx)[2]) {
+        constexpr bool EXP = decltype(has_exp)::value;
+        float f[2][4];
+        if (EXP)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) f[i >> 2][i & 3] = blk_unscale(kx[i >> 2], i & 3);
 #pragma unroll
         for (int ni = 0; ni < 4; ++ni)
 #pragma unroll
             for (int mm = 0; mm < 2; ++mm)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float o = acc[half * 2 + mm][ni][r];
-                    acc[half * 2 + mm][ni][r] =
-                        W::kMin ? fmaf(dv[ni], t[mm][ni][r], fmaf(mv[ni], ts[mm][r], o)) : fmaf(dv[ni], t[mm][ni][r], o);
+                    float o = acc[half * 2 + mm][ni][r];
+                    if (W::kMin) o = fmaf(mv[ni], EXP ? f[mm][r] * ts[mm][r] : ts[mm][r], o);
+                    acc[half * 2 + mm][ni][r] = fmaf(dv[ni], EXP ? f[mm][r] * t[mm][ni][r] : t[mm][ni][r], o);
                 }
     };
     const h8_t ones = {1, 1, 1, 1, 1, 1, 1, 1};
-    auto compute = [&](int buf, int blk, bool pending) {
+    auto compute = [&](auto has_exp, int buf, int blk, bool pending) {
         const h8_t* st = (const h8_t*)(lds + buf * kBigStageBytes);
         const unsigned char* sb = lds + buf * kBigStageBytes + kBigABytes;
         const uint32_t* sd = (const uint32_t*)(lds + buf * kBigStageBytes + kBigABytes + kBigBBytes);
@@ -865,10 +1020,10 @@ __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a)
             if constexpr (W::kPair) {
                 dv[ni] = h2f(((const uint16_t*)dtab)[(blk / 8 - s0 / 8) * 256 + qb[ni] * 16 + l16]);
                 mv[ni] = 0.0f;
-                W::cvt(W::lds(sb + qb[ni] * W::kSub, sb + kBigHiOff + qb[ni] * 128, l16, lc), sd[qb[ni] * 16 + l16],
+                W::cvt(W::lds(sb + qb[ni] * W::kSub, sb + kBigHiOff + qb[ni] * 128, l16, lc), sd[sq[ni]],
                        blk & 1, lc, bh[ni], bl[ni]);
             } else {
-                pf_scale<W::kScale>(W::kScale ? sd[qb[ni] * 16 + l16] : 0u, blk, dv[ni], mv[ni]);
+                pf_scale<W::kScale>(W::kScale ? sd[sq[ni]] : 0u, blk, dv[ni], mv[ni]);
                 bh[ni] = W::cvt(W::lds(sb + qb[ni] * W::kSub, l16, lc), lc);
             }
         }
@@ -905,9 +1060,16 @@ __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a)
         };
         f4_t t0[2][4], ts0[2];
         mfmas(0, t0, ts0);
-        if (pending) scale_in(1, tp, tsp, dvp, mvp);
+        if (pending) scale_in(has_exp, 1, tp, tsp, dvp, mvp, kxp);
         mfmas(1, tp, tsp);
-        scale_in(0, t0, ts0, dv, mv);
+        uint32_t kx[2];
+        if (decltype(has_exp)::value)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                kx[i] = sd[(wm * 4 + i) * (kBigScaleBytes / 4) + 32 + lc];
+                kxp[i] = sd[(wm * 4 + 2 + i) * (kBigScaleBytes / 4) + 32 + lc];
+            }
+        scale_in(has_exp, 0, t0, ts0, dv, mv, kx);
 #pragma unroll
         for (int ni = 0; ni < 4; ++ni) {
             dvp[ni] = dv[ni];
@@ -916,22 +1078,34 @@ __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a)
     };
 
     const int pre = S < kBigStages - 1 ? S : kBigStages - 1;
-    for (int s = 0; s < pre; ++s) issue(s);
-    for (int s = 0; s < S; ++s) {
-        // this wave's loads of stage s are done when at most those of the (up to two) stages
-        // issued after it are in flight; the barrier then makes every wave's done, and every
-        // wave has left compute(s - 1), whose buffer stage s + 3 takes
-        const int after = S - 1 - s;
-        if (after >= 2)
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * kLoads) : "memory");
-        else if (after == 1)
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kLoads) : "memory");
-        else
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if (s + kBigStages - 1 < S) issue(s + kBigStages - 1);
-        compute(s % kBigStages, s0 + s, s > 0);
-    }
-    if (S > 0) scale_in(1, tp, tsp, dvp, mvp);
+    auto run = [&](auto has_exp) {  // the first `pre` stages are issued
+        constexpr bool EXP = decltype(has_exp)::value;
+        constexpr int L = kLoads + (EXP && !W::kScale ? 1 : 0);
+        if (EXP)
+            for (int s = 0; s < pre; ++s) issue_exps(s);
+        for (int s = 0; s < S; ++s) {
+            // this wave's loads of stage s are done when at most those of the (up to two) stages
+            // issued after it are in flight (the first stages' exponents came after all of them); the
+            // barrier then makes every wave's done, and every wave has left compute(s - 1), whose
+            // buffer stage s + 3 takes
+            const int after = EXP && s == 0 ? 0 : S - 1 - s;
+            if (after >= 2)
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * L) : "memory");
+            else if (after == 1)
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(L) : "memory");
+            else
+                asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if (s + kBigStages - 1 < S) issue(has_exp, s + kBigStages - 1);
+            compute(has_exp, s % kBigStages, s0 + s, s > 0);
+        }
+        if (S > 0) scale_in(has_exp, 1, tp, tsp, dvp, mvp, kxp);
+    };
+    const bool exps = MODE == GEMV_RESID && has_exps(a, mt * kBigRows);
+    for (int s = 0; s < pre; ++s) issue(std::false_type{}, s);
+    if (exps)
+        run(std::true_type{});
+    else
+        run(std::false_type{});
 
     if constexpr (SILU && !SPLIT) {
         // silu(gate) * up through LDS (this wave's 64 rows x 32 columns, one block of the next
@@ -956,14 +1130,19 @@ __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a)
         }
         const int blk = a.hid_col0 / 32 + u0 / 2;
         h8_t* out = (h8_t*)a.hid;
+        bool any = false;
 #pragma unroll
         for (int mi = 0; mi < 4; ++mi) {
             const int tile = mt * 8 + wm * 4 + mi, row = 16 * tile + l16;
             const int e = row < a.M ? hid_exp(a, row) : 0;
-            const float sc = ldexpf(1.0f, e);
             const float* src = hl + (16 * mi + l16) * kLd + 8 * lc;
             const float4 x0 = *(const float4*)src, x1 = *(const float4*)(src + 4);
             const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+            float m = 0.0f;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) m = fmaxf(m, fabsf(x[k]));
+            const int kx = row < a.M ? blk_exp(max_of_4(m), e) : 0;
+            const float sc = ldexpf(1.0f, e + kx);
             h8_t hi, lo;
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
@@ -974,8 +1153,11 @@ __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a)
             h8_t* o = out + ((int64_t)tile * a.hid_nblk + blk) * 128 + lane;
             o[0] = hi;
             o[64] = lo;
+            if (lc == 0) a.hid_kx[(int64_t)blk * a.Mpad + row] = (int8_t)kx;
             if (u0 == 0 && lc == 0) a.hid_rs[row] = ldexpf(1.0f, -e);
+            any |= kx != 0;
         }
+        if (__builtin_amdgcn_ballot_w64(any) != 0 && lane == 0) a.hid_kxf[mt] = 1;
         return;
     }
     // epilogue: lane holds rows 16 T + 4 (lane / 16) + r of weight column 16 q + l16
@@ -1061,8 +1243,10 @@ __global__ __launch_bounds__(kBlock) void k_pf_reduce(const PfGemmArgs a) {
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = (v[e] / (1.0f + expf(-v[e]))) * w[e];
-        const int ex = hid_exp(a, row);
-        const float sc = ldexpf(1.0f, ex);
+        // the block's other 28 columns are with the 7 lanes beside this one
+        float m = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+        const int ex = hid_exp(a, row), kx = blk_exp(max_of_8(m), ex);
+        const float sc = ldexpf(1.0f, ex + kx);
         h4_t hi, lo;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -1073,6 +1257,10 @@ __global__ __launch_bounds__(kBlock) void k_pf_reduce(const PfGemmArgs a) {
         _Float16* o = hid_at(a, row, col0);
         *(h4_t*)o = hi;
         *(h4_t*)(o + 512) = lo;
+        if (col0 % 32 == 0) {
+            *hid_kx_at(a, row, col0) = (int8_t)kx;
+            if (kx != 0) a.hid_kxf[row / 128] = 1;
+        }
         if (col0 == 0) a.hid_rs[row] = ldexpf(1.0f, -ex);
         return;
     }
@@ -1359,6 +1547,8 @@ __global__ __launch_bounds__(kBlock) void k_pf_pack_kv(const float* kc, const fl
                                                        int max_seq, int key0, int n_keys, unsigned char* recs,
                                                        const PfAttnOperand op) {
     constexpr int NC = HD / 32;
+    for (int i = (blockIdx.y * gridDim.x + blockIdx.x) * kBlock + threadIdx.x; i < op.n_clear; i += gridDim.x * gridDim.y * kBlock)
+        op.clear[i] = 0;
     __shared__ float ks[kAttnTile][HD + 1], vs[kAttnTile][HD + 1];
     __shared__ int ex[2][kAttnTile];
     const int t = blockIdx.x, g = blockIdx.y, tid = threadIdx.x;
@@ -2046,7 +2236,8 @@ hipError_t launch_pf_gemm(const PfGemmArgs& a, hipStream_t st, bool* fused) {
         if (a.mode == GEMV_SILU && (g.w2.type != t || g.w2.K != a.K || g.w2.N != g.w.N)) return hipErrorInvalidValue;
     }
     if (a.seg[0].sub0 != 0 || (a.mode == GEMV_SILU && a.n_seg != 1)) return hipErrorInvalidValue;
-    if (a.mode == GEMV_SILU && (!a.hid || !a.hid_rs || !a.xn || !a.wn_gate || !a.wn_up || a.hid_col0 % 32 != 0 || a.n_sub % 2 != 0))
+    if (!a.kx != !a.kxf) return hipErrorInvalidValue;
+    if (a.mode == GEMV_SILU && (!a.hid || !a.hid_rs || !a.hid_kx || !a.hid_kxf || !a.xn || !a.wn_gate || !a.wn_up || a.hid_col0 % 32 != 0 || a.n_sub % 2 != 0))
         return hipErrorInvalidValue;
     if (t == TF_HIP_TYPE_F32) {
         // register-streamed tiles only: 4 column subtiles per wave, 2 when that leaves

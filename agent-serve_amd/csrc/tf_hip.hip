@@ -93,6 +93,8 @@ struct tf_hip_ctx {
     int pf_cap = 0;                    // rows per prefill chunk (multiple of kPfTileM)
     float *px = nullptr, *pqkv = nullptr, *ph = nullptr, *prs = nullptr;
     float *phrs = nullptr, *pxn = nullptr;  // ph's row scales as an operand; sums of squares of the FFN's input rows
+    int8_t* pkx = nullptr;                  // ph's block exponents
+    uint32_t* pkxf = nullptr;               // and their flags
     float* pvmax = nullptr;                 // largest value element of an attention call: two words, used in turn
     int pvmax_i = 0;                        // the word that is 0 now
     float* row_norms = nullptr;             // largest row norm of each layer's ffn_gate and ffn_up [layer][2]
@@ -662,7 +664,8 @@ int ensure_pf(tf_hip_ctx* c) {
         if ((rc = dalloc(c, &c->px, cap * D * 4)) || (rc = dalloc(c, &c->pqkv, cap * NQ * 4)) ||
             (rc = dalloc(c, &c->ph, cap * F * 4)) || (rc = dalloc(c, &c->prs, (size_t)cap * 4)) ||
             (rc = dalloc(c, &c->pxa, cap * kmax * 2 * 2)) || (rc = dalloc(c, &c->pvmax, 2 * sizeof(float))) ||
-            (rc = dalloc(c, &c->phrs, (size_t)cap * 4)) || (rc = dalloc(c, &c->pxn, (size_t)cap * 4)))
+            (rc = dalloc(c, &c->phrs, (size_t)cap * 4)) || (rc = dalloc(c, &c->pxn, (size_t)cap * 4)) ||
+            (rc = dalloc(c, &c->pkx, cap * (F / 32))) || (rc = dalloc(c, &c->pkxf, (size_t)(cap / 128) * 4)))
             return rc;
         // up to 8 K slices of the widest non-SILU output (QKV or d_model)
         c->ppart_floats = 8 * (size_t)cap * std::max(NQ, D);
@@ -950,7 +953,8 @@ int prefill_mfma(tf_hip_ctx* c, int n) {
                 if (last) chk(prefill_last_row(c, l, c->pqkv + (int64_t)(nc - 1) * NQ, nc, start + n - 1, start));
                 continue;
             }
-            const PfAttnOperand op{c->pxa, c->prs, c->pvmax + c->pvmax_i, c->pvmax + (c->pvmax_i ^ 1)};
+            const PfAttnOperand op{c->pxa, c->prs, c->pvmax + c->pvmax_i, c->pvmax + (c->pvmax_i ^ 1),
+                                   c->pkxf, (Mpad + 127) / 128};
             c->pvmax_i ^= 1;
             chk(launch_pf_attn(c->pqkv, NQ, kc, vc, p.kv_layout, p.n_head, p.n_kv_head, p.head_dim, p.max_seq, nc,
                                pos0, start, nullptr, 0, c->pattn_ws, c->pattn_ws_bytes, c->st, op));
@@ -987,6 +991,8 @@ int prefill_mfma(tf_hip_ctx* c, int n) {
                     a.n_sub = (c1 - c0) / 16;
                     a.hid = (uint16_t*)c->ph;  // 4 bytes an element either way
                     a.hid_rs = c->phrs;
+                    a.hid_kx = c->pkx;
+                    a.hid_kxf = c->pkxf;
                     a.hid_col0 = c0;
                     a.hid_nblk = F / 32;
                     a.xn = c->pxn;
@@ -1011,6 +1017,8 @@ int prefill_mfma(tf_hip_ctx* c, int n) {
                 if (!h_split) {  // the hidden rows came out as an operand in ph
                     a.xa = (const uint16_t*)c->ph;
                     a.rs = c->phrs;
+                    a.kx = c->pkx;
+                    a.kxf = c->pkxf;
                 }
                 a.mode = GEMV_RESID;
                 seg(a, M(TF_HIP_LAYER_DOWN), c->px, D, nullptr);

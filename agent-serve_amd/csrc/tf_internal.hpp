@@ -178,6 +178,10 @@ struct PfSeg {
 struct PfGemmArgs {
     const uint16_t* xa = nullptr;  // [Mpad/16][K/32][hi, lo][64][8] fp16 (fragment order)
     const float* rs = nullptr;     // [Mpad] row scales
+    // GEMV_RESID, for an operand with block exponents (nullptr: all 0): row m's block b holds 2^kx times
+    // what rs says, kx[b][Mpad] at m; kxf[m / 128] is not 0 where one of 128 rows has one that is not 0
+    const int8_t* kx = nullptr;
+    const uint32_t* kxf = nullptr;
     int K = 0, M = 0, Mpad = 0;
     PfSeg seg[3];
     int n_seg = 0;
@@ -198,12 +202,15 @@ struct PfGemmArgs {
     const float* split_w = nullptr;
     float split_eps = 0.0f;
     float* split_xn = nullptr;     // GEMV_RESID: the split rows' sums of squares, when wanted
-    // GEMV_SILU: the silu * up rows go out as the next GEMM's operand (hid, its row scales hid_rs),
-    // columns from hid_col0 on of hid_nblk blocks a row; scaled by a bound from the input rows' sums
-    // of squares xn and the largest norms of a gate and of an up row (launch_row_norm_max). A
-    // K-split reduce with split_xa set splits them there by their largest value instead.
+    // GEMV_SILU: the silu * up rows go out as the next GEMM's operand (hid, its row scales hid_rs, its
+    // block exponents hid_kx and their flags hid_kxf, 0 before the launch), columns from hid_col0 on of
+    // hid_nblk blocks a row; the row scales come from the input rows' sums of squares xn and the largest
+    // norms of a gate and of an up row (launch_row_norm_max). A K-split reduce with split_xa set splits
+    // them there by their largest value instead.
     uint16_t* hid = nullptr;
     float* hid_rs = nullptr;
+    int8_t* hid_kx = nullptr;
+    uint32_t* hid_kxf = nullptr;
     int hid_col0 = 0, hid_nblk = 0;
     const float *xn = nullptr, *wn_gate = nullptr, *wn_up = nullptr;
     // GEMV_STORE of the q, k and v segments, rope_cos set: launch_pf_rope_store of the rows
@@ -276,6 +283,8 @@ struct PfAttnOperand {
     uint16_t* xa = nullptr;
     float* rs = nullptr;
     float *vmax = nullptr, *vmax_next = nullptr;
+    uint32_t* clear = nullptr;  // n_clear words that the launch sets to 0: the hidden rows' exponent flags
+    int n_clear = 0;
 };
 // Workspace of launch_pf_attn for attention over n_keys positions: the packed key/value
 // tile records.

@@ -260,9 +260,10 @@ SHORT_PROMPT_MODELS = [
 
 class RawModel:
     """A two-layer context built through the C ABI from rows(rng, slot, type, k, n), with the same
-    model in float64. fmts: formats of q, k, v, o, gate / up, down."""
+    model in float64. fmts: formats of q, k, v, o, gate / up, down. edit(slot, v) changes a norm's weights
+    or a bias in place."""
 
-    def __init__(self, pkg, heads, kv, d, ff, fmts, max_seq, rows):
+    def __init__(self, pkg, heads, kv, d, ff, fmts, max_seq, rows, edit=lambda slot, v: None):
         import ctypes as C
 
         from gpu_util import oracle_dequant
@@ -281,6 +282,7 @@ class RawModel:
 
         def vec(slot, n, mean):
             v = (mean + 0.2 * rng.standard_normal(n)).astype(np.float32)
+            edit(slot, v)
             self.w[slot] = v.astype(np.float64)
             assert L.tf_hip_upload_tensor(self.ctx, slot, 0, n, 1, v.ctypes.data, v.nbytes) == 0
 
@@ -384,8 +386,9 @@ def test_short_prompt_kernels(pkg, shape):
 @pytest.mark.parametrize("t", [8, 3, 1, 14, 0])
 @pytest.mark.parametrize("ff,n", [(512, 70), (4096, 130), (16384, 250)])
 def test_hidden_rows_scaled_by_a_bound(pkg, t, ff, n):
-    """ffn_down's operand is scaled by a bound from the gate and up rows' norms: rows of 2^-5 to 2^5 times
-    the others (one in 16) loosen it to 2^14 above most hidden values. The K-split reduce, the
+    """ffn_down's operand has its row scales from the gate and up rows' norms: rows of 2^-5 to 2^5 times the
+    others (one in 16) put that bound up to 2^14 above most hidden values, inside and outside of what
+    needs block exponents (test_hidden_rows_of_uneven_models goes further). The K-split reduce, the
     streamed tiles and the large ones (16,384 hidden units at 250 rows: unsplit) write it. Against
     float64 within the 2e-5 of the other model tests: scaled by the rows' largest values, the same
     models measured up to 1.3e-5 (Q4_1 at 512 hidden units, whose two terms cancel) and 8e-6."""
@@ -400,6 +403,58 @@ def test_hidden_rows_scaled_by_a_bound(pkg, t, ff, n):
         tokens = np.random.default_rng(n).integers(0, m.vocab, n).astype(np.int32)
         for a, e in zip(m.prefill(MFMA, tokens), m.exact(tokens)):
             assert rel_err(a, e) <= 2e-5
+    finally:
+        m.close()
+
+
+# format, d_model, ffn, prompt, kind (not Q4_1's input channel: its two terms cancel there, in gate and up
+# themselves)
+UNEVEN_MODELS = [(t, d, ff, n, kind)
+                 for d, ff, n in ((256, 512, 70), (256, 4096, 130), (256, 8192, 500), (64, 512, 10), (64, 512, 20), (64, 128, 60))
+                 for t in ((8, 3, 1, 14, 0) if d == 256 else (8, 3, 1, 0))
+                 for kind in ("rows_8", "rows_10", "silu", "channel") if t != 3 or kind != "channel"]
+
+
+@pytest.mark.parametrize("t,d,ff,n,kind", UNEVEN_MODELS)
+def test_hidden_rows_of_uneven_models(pkg, t, d, ff, n, kind):
+    """ffn_down's operand keeps its bits where the norms of the gate and up rows say little about the hidden
+    values: one gate row and another unit's up row 2^8 or 2^10 times the others, ffn_down reading
+    neither; one unit with a gate so far below 0 that its silu is 0, its up row 2^12 times the others;
+    an input channel 2^12 times the others that the weights hardly use. The products of the norms
+    are 2^25 to 2^33 above the hidden values. The K-split reduce, the streamed tiles (of 16, 32 and 64
+    rows, K split or not) and the large ones (500 rows) write and read it; a V matrix in F32 keeps
+    prompts of at most 16 tokens on them. The tolerance is check()'s."""
+    def rows(rng, slot, t, k, n):
+        w = (rng.standard_normal((n, k)) / np.sqrt(k)).astype(np.float32)
+        which = (slot - 16) % 12 if slot >= 16 else -1
+        if kind.startswith("rows"):
+            if which == 9:
+                w[5] *= 2.0 ** int(kind[5:])
+            if which == 10:
+                w[(n // 2 + 40) % n] *= 2.0 ** int(kind[5:])
+            if which == 11:
+                w[:, [5, (k // 2 + 40) % k]] = 0.0
+        if kind == "silu":
+            if slot == 0:
+                w[:, 0] = 0.25
+            if which == 9:
+                w[5] = 0.0
+                w[5, 0] = -4096.0
+            if which == 10:
+                w[5] *= 4096.0
+            if which in (4, 11):
+                w[0] = 0.0  # the residual rows keep their first element
+        if kind == "channel" and which in (9, 10):
+            w[:, 0] /= 4096.0
+        return np.stack([pkg.quantize_row(t, r) for r in w])
+
+    def edit(slot, v):
+        if kind == "channel" and slot >= 16 and (slot - 16) % 12 == 8:
+            v[0] = 4096.0
+
+    m = RawModel(pkg, d // 32, d // 64, d, ff, (t, t, 0 if n <= 16 else t, t, t, t), 512, rows, edit)
+    try:
+        m.check(np.random.default_rng(n).integers(0, m.vocab, n).astype(np.int32))
     finally:
         m.close()
 
