@@ -336,8 +336,9 @@ __global__ __launch_bounds__(kBlock) void k_pf_split(const float* x, int64_t ldx
 // Field of the segment holding output subtile u (uniform per wave: scalar selects).
 #define PF_SEL(s, f) ((s) == 0 ? a.seg[0].f : ((s) == 1 ? a.seg[1].f : a.seg[2].f))
 
-// An operand whose rows no workgroup has whole (the hidden rows): the row scale is 2^-e for an e
-// that a bound gives, and each 32-element block has an exponent kx of its own, so that how loose the bound is costs no bits. A block whose largest value m gives 2^4 <= m 2^e < 2^15 is
+// An operand whose rows no workgroup has whole (the attention output, the hidden rows): the row scale is
+// 2^-e for an e that a bound gives, and each 32-element block has an exponent kx of its own, so that
+// how loose the bound is costs no bits. A block whose largest value m gives 2^4 <= m 2^e < 2^15 is
 // written as v 2^e (kx 0): fp16's pair hi + lo keeps 22 bits of what is at least 2^-7 of m, and the
 // rest to 2^-29 of m. Any other block is written as v 2^(e + kx), m 2^(e + kx) in [2^14, 2^15). The GEMM
 // takes 2^kx out of the block's sum, an exact operation, in a loop of its own that runs where a flag
@@ -1575,7 +1576,7 @@ __global__ __launch_bounds__(kBlock) void k_pf_pack_kv(const float* kc, const fl
         if (part == 0) ex[which][key] = m > 0.0f ? pow2_exp(m, 0) : kZeroRow;
         if (op.xa) {
             // the largest finite value element (an infinite one makes the rows that see it NaN whatever
-            // their scale, and the others do not depend on it), for the output's scale
+            // their scale, and the others do not depend on it), for the output's row scales
             const float mv = wave_max(which && m < INFINITY ? m : 0.0f);
             if (which && (tid & 63) == 0) atomicMax((int*)op.vmax, __float_as_int(mv));
             if (t == 0 && g == 0 && tid == 0) *op.vmax_next = 0.0f;
@@ -1911,31 +1912,47 @@ __global__ __launch_bounds__(512) void k_pf_attn(const float* q, int64_t ldq, co
         if (qi >= n) continue;
         const float il = ldexpf(1.0f / l_run[qs], -unit[qs]);
         if (op.xa) {
-            // as wo's operand: an output is a mean of values, so no larger than the largest of
-            // them (2^ex of it with a bit to spare for rounding) and every row has that scale.
-            // Against fp32 rows and a pass to split them (5 us a layer at 512 rows): 333 tokens of
-            // the 4-bit Llama-3.2-1B shape 3.54 -> 3.50 ms, 2,900 of the Qwen2.5-1.5B shape 1 %.
+            // as wo's operand: an output is a mean of values, so no larger than the largest of them
+            // (2^ex bounds it), which gives every row's scale; the blocks have exponents, for heads
+            // and rows that see smaller values only. Against fp32 rows and a pass to split them (5 us
+            // a layer at 512 rows): 333 tokens of the 4-bit Llama-3.2-1B shape 3.54 -> 3.50 ms, 2,900
+            // of the Qwen2.5-1.5B shape 1 %.
             int ex;
             (void)frexpf(*op.vmax, &ex);
-            int e = 14 - ex;
+            int e = 15 - ex;
             e = e < -100 ? -100 : (e > 100 ? 100 : e);
-            const float sc = ldexpf(1.0f, e);
+            int any = 0;
 #pragma unroll
-            for (int d = 0; d < NT; ++d) {
-                const int col = h * HD + 16 * d + 4 * gq;
-                h4_t hi, lo;
+            for (int b = 0; b < NT / 2; ++b) {  // 32 columns
+                const int col0 = h * HD + 32 * b;
+                float m = 0.0f, v[2][4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float t = acc[qs][d][r] * il * sc;
-                    hi[r] = (_Float16)t;
-                    lo[r] = (_Float16)(t - (float)hi[r]);
+                for (int i = 0; i < 8; ++i) {
+                    v[i >> 2][i & 3] = acc[qs][2 * b + (i >> 2)][i & 3] * il;
+                    m = fmaxf(m, fabsf(v[i >> 2][i & 3]));
                 }
-                _Float16* o = (_Float16*)op.xa +
-                              (((int64_t)(qi / 16) * (G * n_rep * HD / 32) + col / 32) * 128 + qi % 16 + 16 * (col % 32 / 8)) * 8 +
-                              col % 8;
-                *(h4_t*)o = hi;
-                *(h4_t*)(o + 512) = lo;
+                const int kx = blk_exp(max_of_4(m), e);
+                const float sc = ldexpf(1.0f, e + kx);
+#pragma unroll
+                for (int d = 0; d < 2; ++d) {
+                    const int cb = 16 * d + 4 * gq;  // column of the block
+                    h4_t hi, lo;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float t = v[d][r] * sc;
+                        hi[r] = (_Float16)t;
+                        lo[r] = (_Float16)(t - (float)hi[r]);
+                    }
+                    _Float16* o = (_Float16*)op.xa +
+                                  (((int64_t)(qi / 16) * (G * n_rep * HD / 32) + col0 / 32) * 128 + qi % 16 + 16 * (cb / 8)) * 8 +
+                                  cb % 8;
+                    *(h4_t*)o = hi;
+                    *(h4_t*)(o + 512) = lo;
+                }
+                if (gq == 0) op.kx[(int64_t)(col0 / 32) * op.kx_ld + qi] = (int8_t)kx;
+                any |= kx;
             }
+            if (any != 0 && gq == 0) op.kxf[qi / 128] = 1;
             if (h == 0 && gq == 0) op.rs[qi] = ldexpf(1.0f, -e);
             continue;
         }
@@ -2329,7 +2346,7 @@ hipError_t launch_pf_attn(const float* q, int64_t ldq, const float* kc, const fl
                           size_t ws_bytes, hipStream_t st, const PfAttnOperand& op) {
     if (n <= 0) return hipSuccess;
     const int n_rep = H / G;
-    if (op.xa && (!op.rs || !op.vmax || !op.vmax_next || H * hd % 32 != 0)) return hipErrorInvalidValue;
+    if (op.xa && (!op.rs || !op.kx || !op.kxf || op.kx_ld < n || !op.vmax || !op.vmax_next || H * hd % 32 != 0)) return hipErrorInvalidValue;
     if (H % G != 0 || !pf_attn_supported(hd, n_rep) || att_start < 0 || att_start > pos0 || pos0 + n > max_seq ||
         ldq % 4 != 0 || ldo % 4 != 0 || !ws || ws_bytes < pf_attn_ws_bytes(hd, G, pos0 + n - att_start))
         return hipErrorInvalidValue;

@@ -93,8 +93,8 @@ struct tf_hip_ctx {
     int pf_cap = 0;                    // rows per prefill chunk (multiple of kPfTileM)
     float *px = nullptr, *pqkv = nullptr, *ph = nullptr, *prs = nullptr;
     float *phrs = nullptr, *pxn = nullptr;  // ph's row scales as an operand; sums of squares of the FFN's input rows
-    int8_t* pkx = nullptr;                  // ph's block exponents
-    uint32_t* pkxf = nullptr;               // and their flags
+    int8_t* pkx = nullptr;                  // block exponents of the attention rows in pxa, then of ph
+    uint32_t* pkxf = nullptr;               // their flags: the attention rows' pf_cap / 128, then ph's
     float* pvmax = nullptr;                 // largest value element of an attention call: two words, used in turn
     int pvmax_i = 0;                        // the word that is 0 now
     float* row_norms = nullptr;             // largest row norm of each layer's ffn_gate and ffn_up [layer][2]
@@ -665,7 +665,8 @@ int ensure_pf(tf_hip_ctx* c) {
             (rc = dalloc(c, &c->ph, cap * F * 4)) || (rc = dalloc(c, &c->prs, (size_t)cap * 4)) ||
             (rc = dalloc(c, &c->pxa, cap * kmax * 2 * 2)) || (rc = dalloc(c, &c->pvmax, 2 * sizeof(float))) ||
             (rc = dalloc(c, &c->phrs, (size_t)cap * 4)) || (rc = dalloc(c, &c->pxn, (size_t)cap * 4)) ||
-            (rc = dalloc(c, &c->pkx, cap * (F / 32))) || (rc = dalloc(c, &c->pkxf, (size_t)(cap / 128) * 4)))
+            (rc = dalloc(c, &c->pkx, cap * (std::max(F, (size_t)c->H) / 32))) ||
+            (rc = dalloc(c, &c->pkxf, (size_t)(cap / 128) * 2 * 4)))
             return rc;
         // up to 8 K slices of the widest non-SILU output (QKV or d_model)
         c->ppart_floats = 8 * (size_t)cap * std::max(NQ, D);
@@ -953,13 +954,16 @@ int prefill_mfma(tf_hip_ctx* c, int n) {
                 if (last) chk(prefill_last_row(c, l, c->pqkv + (int64_t)(nc - 1) * NQ, nc, start + n - 1, start));
                 continue;
             }
-            const PfAttnOperand op{c->pxa, c->prs, c->pvmax + c->pvmax_i, c->pvmax + (c->pvmax_i ^ 1),
-                                   c->pkxf, (Mpad + 127) / 128};
+            const PfAttnOperand op{c->pxa, c->prs,  c->pvmax + c->pvmax_i, c->pvmax + (c->pvmax_i ^ 1),
+                                   c->pkx, Mpad,    c->pkxf,               c->pkxf,
+                                   2 * (c->pf_cap / 128)};
             c->pvmax_i ^= 1;
             chk(launch_pf_attn(c->pqkv, NQ, kc, vc, p.kv_layout, p.n_head, p.n_kv_head, p.head_dim, p.max_seq, nc,
                                pos0, start, nullptr, 0, c->pattn_ws, c->pattn_ws_bytes, c->st, op));
             {
                 PfGemmArgs a = base(Hd);
+                a.kx = c->pkx;
+                a.kxf = c->pkxf;
                 a.mode = GEMV_RESID;
                 seg(a, M(TF_HIP_LAYER_O), c->px, D, nullptr);
                 fuse_split(a, V(TF_HIP_LAYER_FFN_NORM));
@@ -992,7 +996,7 @@ int prefill_mfma(tf_hip_ctx* c, int n) {
                     a.hid = (uint16_t*)c->ph;  // 4 bytes an element either way
                     a.hid_rs = c->phrs;
                     a.hid_kx = c->pkx;
-                    a.hid_kxf = c->pkxf;
+                    a.hid_kxf = c->pkxf + c->pf_cap / 128;
                     a.hid_col0 = c0;
                     a.hid_nblk = F / 32;
                     a.xn = c->pxn;
@@ -1018,7 +1022,7 @@ int prefill_mfma(tf_hip_ctx* c, int n) {
                     a.xa = (const uint16_t*)c->ph;
                     a.rs = c->phrs;
                     a.kx = c->pkx;
-                    a.kxf = c->pkxf;
+                    a.kxf = c->pkxf + c->pf_cap / 128;
                 }
                 a.mode = GEMV_RESID;
                 seg(a, M(TF_HIP_LAYER_DOWN), c->px, D, nullptr);

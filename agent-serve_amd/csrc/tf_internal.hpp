@@ -276,14 +276,17 @@ hipError_t launch_pf_rope_store(float* qkv, int64_t ld, int n, int H, int G, int
                                 const float* rope_sin, int pos0, float* kc, float* vc, int layout, int max_seq,
                                 hipStream_t st);
 bool pf_attn_supported(int hd, int n_rep);
-// Where launch_pf_attn writes its rows as the next GEMM's operand (xa, row scales rs) instead of
-// as floats: vmax is 0 before the launch and takes the largest value element; vmax_next is set to 0
-// for the launch after.
+// Where launch_pf_attn writes its rows as the next GEMM's operand (xa, row scales rs, block exponents
+// kx [H / 32][kx_ld] and their flags kxf) instead of as floats: vmax is 0 before the launch and
+// takes the largest value element; vmax_next is set to 0 for the launch after.
 struct PfAttnOperand {
     uint16_t* xa = nullptr;
     float* rs = nullptr;
     float *vmax = nullptr, *vmax_next = nullptr;
-    uint32_t* clear = nullptr;  // n_clear words that the launch sets to 0: the hidden rows' exponent flags
+    int8_t* kx = nullptr;
+    int kx_ld = 0;
+    uint32_t* kxf = nullptr;
+    uint32_t* clear = nullptr;  // n_clear words set to 0 before the rows are written: these flags and the hidden rows'
     int n_clear = 0;
 };
 // Workspace of launch_pf_attn for attention over n_keys positions: the packed key/value

@@ -459,6 +459,35 @@ def test_hidden_rows_of_uneven_models(pkg, t, d, ff, n, kind):
         m.close()
 
 
+@pytest.mark.parametrize("heads,kv,t,n", [(4, 2, 8, 70), (2, 1, 3, 130), (8, 2, 14, 250), (4, 4, 1, 250), (4, 2, 0, 70)])
+def test_attention_rows_of_uneven_values(pkg, heads, kv, t, n):
+    """wo's operand keeps its bits in the rows that see small values only: the prompt's last token alone has
+    a value element some 2^23 times the others'. K and V rows of the second layer (behind the
+    first one's attention) of the tokens before it, no further from float64 than twice the per-token
+    path's, or 4e-6 where that is closer still."""
+    def rows(rng, slot, t, k, n):
+        w = (rng.standard_normal((n, k)) / np.sqrt(k)).astype(np.float32)
+        if slot == 0:
+            w[:, 0] = 0.0
+            w[n - 1, 0] = 1.0
+        if slot == 16 + 3:
+            w[3, 0] = 2.0 ** 20
+        return np.stack([pkg.quantize_row(t, r) for r in w])
+
+    m = RawModel(pkg, heads, kv, 256, 512, (t, t, 0, t, t, t), 256, rows)
+    try:
+        tokens = np.random.default_rng(n).integers(0, m.vocab - 1, n).astype(np.int32)
+        tokens[-1] = m.vocab - 1
+        want, got, again = (m.prefill(p, tokens) for p in (TOKENS, MFMA, MFMA))
+        for i, e in enumerate(m.exact(tokens)):
+            assert np.array_equal(got[i].view(np.uint32), again[i].view(np.uint32)), i
+            if i in (5, 6):
+                b, a, e = got[i][:-1], want[i][:-1], e[:-1]
+                assert rel_err(b, e) <= max(2 * rel_err(a, e), 4e-6), (i, rel_err(b, e), rel_err(a, e))
+    finally:
+        m.close()
+
+
 # type, query heads, kv heads, d_model, ffn, max_seq, prompt: rows shorter and longer than a tile, rows
 # that do not fill one (192, 320), head sizes 32, 64 and 128, odd ffn row counts for the row groups,
 # attention on one workgroup per kv head and split over workgroups
