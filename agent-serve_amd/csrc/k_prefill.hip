@@ -1129,6 +1129,9 @@ __global__ __launch_bounds__(kBigThreads) void k_pf_gemm_big(const PfGemmArgs a)
                     hl[(16 * mi + 4 * (lane >> 4) + r) * kLd + 16 * ni + l16] = (gv / (1.0f + expf(-gv))) * uv;
                 }
         }
+        // a wave's own rows: its LDS operations keep their order, which the compiler has to keep too
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
         const int blk = a.hid_col0 / 32 + u0 / 2;
         h8_t* out = (h8_t*)a.hid;
         bool any = false;
