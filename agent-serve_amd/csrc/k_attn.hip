@@ -327,7 +327,8 @@ int attn_splits(int max_seq) {
 
 hipError_t launch_attn_decode(const AttnArgs& args, hipStream_t st) {
     AttnArgs a = args;
-    if (a.hd > kCombThreads) return hipErrorInvalidValue;
+    // the tables are read without RoPE too (row 0)
+    if (a.hd > kCombThreads || !a.rope_cos || !a.rope_sin) return hipErrorInvalidValue;
     // a known position: only the splits it fills (split_of's cut of the same positions does not
     // change; a 4096-position cache would launch 128 workgroups a kv head for 32 with work)
     if (a.fixed_pos >= 0) a.S = std::min(a.S, (a.fixed_pos + 1 - a.fixed_start + kAttnMinChunk - 1) / kAttnMinChunk);
