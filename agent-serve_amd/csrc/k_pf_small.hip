@@ -698,7 +698,7 @@ hipError_t launch_small_m(const PfSmallArgs& a, hipStream_t st) {
 hipError_t launch_pf_small(const PfSmallArgs& a, hipStream_t st) {
     if (a.K % 64 != 0 || a.M <= 0 || a.M > kPfSmallRows || a.n_sub <= 0 || a.n_seg < 1 || a.n_seg > 3 || !a.xa ||
         (a.mode != GEMV_RESID && !a.ssp) || (a.oxa && (a.n_seg != 1 || a.n_sub % 2 != 0)) || (a.onorm_w && !a.ossp) ||
-        (a.mode == GEMV_SILU && !a.oxa))
+        (a.mode == GEMV_SILU && !a.oxa) || (a.part && (!a.count || a.part_floats < kPfSmallPart((size_t)a.n_sub * 16))))
         return hipErrorInvalidValue;
     const int t = a.seg[0].w.type;
     for (int s = 0; s < a.n_seg; ++s) {

@@ -632,6 +632,9 @@ int run_tokens(tf_hip_ctx* c, int* use_step, int n, int greedy, int lm_every, in
     return 0;
 }
 
+// Floats of ppart that prefill_small's sums of squares take: a double a row and 16 columns.
+size_t pf_small_ssp(size_t D) { return 2 * kPfSmallRows * (D / 16); }
+
 // Decides once, after every tensor is uploaded, whether prompts run on the matrix
 // cores: every layer matrix in a format k_pf_gemm handles with row lengths it tiles,
 // and a head size and GQA ratio k_pf_attn handles. Allocates the chunk buffers.
@@ -671,6 +674,10 @@ int ensure_pf(tf_hip_ctx* c) {
         // up to 8 K slices of the widest non-SILU output (QKV or d_model)
         c->ppart_floats = 8 * (size_t)cap * std::max(NQ, D);
         if ((rc = dalloc(c, &c->ppart, c->ppart_floats * 4))) return rc;
+        // prefill_small's two operands lie in pxa, its sums of squares and its slices in ppart
+        if (kPfSmallOperand(D) + kPfSmallOperand(std::max(F, (size_t)c->H)) > cap * kmax * 2 ||
+            pf_small_ssp(D) + kPfSmallPart(D) > c->ppart_floats)
+            c->pf_small = false;
         const size_t count_bytes = D / 16 * sizeof(int);
         if ((rc = dalloc(c, &c->pf_count, count_bytes))) return rc;
         HIPCHK(c, hipMemset(c->pf_count, 0, count_bytes));
@@ -712,11 +719,11 @@ int prefill_small(tf_hip_ctx* c, int n) {
     const tf_hip_hparams& p = c->hp;
     const int D = p.n_embd, F = p.n_ff, Hd = c->H, KVd = c->KVd, NQ = Hd + 2 * KVd;
     // the residual rows' operand, then that of the attention output or the hidden rows; their
-    // sums of squares where longer prompts keep K slices (ensure_pf sized both for 128 rows)
+    // sums of squares where longer prompts keep K slices (ensure_pf checks that they fit)
     uint16_t* xa = c->pxa;
     uint16_t* ha = c->pxa + kPfSmallOperand((size_t)D);
     double* ssp = (double*)c->ppart;
-    float* part = c->ppart + 2 * kPfSmallRows * (size_t)(D / 16);
+    float* part = c->ppart + pf_small_ssp((size_t)D);
     hipError_t e = launch_embed_rows(mat(c, TF_HIP_SLOT_TOKEN_EMBD), c->hist + c->pos, n, c->px, D, c->st);
     auto chk = [&](hipError_t r) {
         if (e == hipSuccess) e = r;
@@ -748,6 +755,7 @@ int prefill_small(tf_hip_ctx* c, int n) {
     };
     auto slices = [&](PfSmallArgs& a) {
         a.part = part;
+        a.part_floats = c->ppart_floats - pf_small_ssp((size_t)D);
         a.count = c->pf_count;
     };
     chk(launch_pf_small_split(c->px, D, n, vec(c, TF_HIP_SLOT_LAYER(0, TF_HIP_LAYER_ATTN_NORM)), xa, ssp, c->st));

@@ -240,9 +240,11 @@ struct PfSmallArgs {
     uint16_t* oxa = nullptr;
     const float* onorm_w = nullptr;
     double* ossp = nullptr;
-    // GEMV_RESID may take K in up to kPfSmallSlices slices: their sums (kPfSmallPart floats) and a
-    // count per tile group (zero before and after every launch), or nullptr
+    // GEMV_RESID may take K in up to kPfSmallSlices slices: their sums (part_floats, at least
+    // kPfSmallPart of the columns) and a count per tile group (zero before and after every launch),
+    // or nullptr
     float* part = nullptr;
+    size_t part_floats = 0;
     int* count = nullptr;
     int ks = 1;  // set by launch_pf_small
 };

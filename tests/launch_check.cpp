@@ -21,5 +21,28 @@ int main() {
     a.rope_cos = nullptr;
     a.rope_sin = row;
     say("attn_cos", launch_attn_decode(a, nullptr));
+
+    // K slices' sums of 256 columns
+    uint16_t half = 0;
+    int count = 0;
+    PfSmallArgs s;
+    s.xa = &half;
+    s.K = 2048;
+    s.M = 1;
+    s.mode = GEMV_RESID;
+    s.n_seg = 1;
+    s.n_sub = 16;
+    s.seg[0].w.type = TF_HIP_TYPE_Q8_0;
+    s.seg[0].w.K = 2048;
+    s.seg[0].w.N = 256;
+    s.seg[0].y = row;
+    s.part = row;
+    s.count = &count;
+    say("small_part", launch_pf_small(s, nullptr));
+    s.part_floats = kPfSmallPart(256) - 1;
+    say("small_part_short", launch_pf_small(s, nullptr));
+    s.part_floats = kPfSmallPart(256);
+    s.count = nullptr;
+    say("small_count", launch_pf_small(s, nullptr));
     return 0;
 }
