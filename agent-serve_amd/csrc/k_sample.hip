@@ -29,6 +29,11 @@
 //   launch_sample       the whole order, where more than kTopCap logits count (flat
 //                       distributions), where a logit is NaN or the maximum infinite, or where
 //                       the caller asks for the order or the probabilities.
+// A call that needs the second after the first pays for both and for the wait between them (about
+// 50 us). With 128,256 logits of deviation 10, by temperature (the logits that count; a whole call by
+// the whole order alone, before k_rs_scan read whole lines, and now): 0.8 (610) 492 -> 54 us, 2 (54,000)
+// 1,140 -> 900, 3 (123,000) 2,940 -> 2,730 to 3,270 -> 3,050 by top_p, 5 (all) 6,170 -> 6,020 to 8,440
+// -> 8,290, 10 (all) 9,080 -> 9,010 to 14,060 -> 13,990: there the sums in order take nearly all of it.
 #include <algorithm>
 
 #include "dev_common.hpp"
@@ -192,48 +197,48 @@ __device__ __forceinline__ void in_order(int n, Val val, Stuck stuck, F f) {
     }
 }
 
-// Steps 3-5 on one wave over p_0 .. p_(n-1) in descending order (the values before any
-// division; a division by s or z is the same float wherever it happens). Returns the place
-// picked, or -1 for the last kept one; `total` is the place count of the whole order,
-// which `last` reads when the nucleus takes everything.
-struct Picked {
-    int place, last;
-    float s, z;
-};
-__device__ __forceinline__ Picked pick(const float* p, int n, int total, float top_p, float r) {
-    Picked o{-1, total, 0.0f, 0.0f};
+// Steps 3-5 on one wave over val(0) .. val(n - 1) in descending order: s; the nucleus (z, and how
+// many values it keeps of `total`, all where the sum stays below top_p); the place of the draw, or -1
+// for the last kept one.
+template <class Val>
+__device__ __forceinline__ float sum_in_order(int n, Val val) {
     float s = 0.0f;
-    in_order(n, [&](int i) { return p[i]; }, [&](float v) { return v <= quarter_ulp(s); },
+    in_order(n, val, [&](float v) { return v <= quarter_ulp(s); },
              [&](int, float v) {
                  s += v;
                  return false;
              });
+    return s;
+}
+template <class Val>
+__device__ __forceinline__ float nucleus(int n, int total, float top_p, int& last, Val val) {
     float acc = 0.0f;
-    if (top_p < 1.0f)
-        in_order(n, [&](int i) { return p[i] / s; }, [&](float v) { return v <= quarter_ulp(acc); },
-                 [&](int i, float v) {
-                     acc += v;
-                     if (acc >= top_p) {
-                         o.last = i + 1;
-                         return true;
-                     }
-                     return false;
-                 });
-    const float z = acc;
-    o.s = s;
-    o.z = z;
-    acc = 0.0f;
-    in_order(min(n, o.last), [&](int i) { return top_p < 1.0f ? p[i] / s / z : p[i] / s; },
-             [&](float v) { return v <= quarter_ulp(acc); },
+    last = total;
+    in_order(n, val, [&](float v) { return v <= quarter_ulp(acc); },
              [&](int i, float v) {
                  acc += v;
-                 if (r <= acc) {
-                     o.place = i;
+                 if (acc >= top_p) {
+                     last = i + 1;
                      return true;
                  }
                  return false;
              });
-    return o;
+    return acc;
+}
+template <class Val>
+__device__ __forceinline__ int draw(int n, float r, Val val) {
+    float acc = 0.0f;
+    int place = -1;
+    in_order(n, val, [&](float v) { return v <= quarter_ulp(acc); },
+             [&](int i, float v) {
+                 acc += v;
+                 if (r <= acc) {
+                     place = i;
+                     return true;
+                 }
+                 return false;
+             });
+    return place;
 }
 
 // Step 2 for the whole order.
@@ -244,24 +249,42 @@ __global__ __launch_bounds__(kBlock) void k_sample_exp(const float* logits, cons
     if (i < n) p[i] = expf_libm((logits[idx[i]] - m) / temperature, kExp2Tab);
 }
 
-// Steps 3-5 for the whole order (one workgroup): the token and, for a caller that asked,
-// the final probabilities in place of p.
+// Steps 3-5 for the whole order (one workgroup): the token, and the final probabilities in place of
+// p. The divisions run on every wave between the sums (on the one wave that adds they took 1.5 % of a
+// nearly flat 128K vocabulary's 14 ms).
 __global__ __launch_bounds__(kSampleThreads) void k_sample(const int32_t* idx, float* p, int n, float top_p, float r,
-                                                           int32_t* out, int want_probs) {
-    __shared__ Picked sh;
-    if (threadIdx.x < 64) {
-        const Picked o = pick(p, n, n, top_p, r);
-        if (threadIdx.x == 0) {
-            *out = idx[o.place >= 0 ? o.place : o.last - 1];
-            sh = o;
-        }
+                                                           int32_t* out) {
+    __shared__ float sh_s, sh_z;
+    __shared__ int sh_last;
+    const int tid = threadIdx.x;
+    const bool w0 = tid < 64;
+    auto val = [&](int i) { return p[i]; };
+    if (w0) {
+        const float s = sum_in_order(n, val);
+        if (tid == 0) sh_s = s;
     }
-    if (!want_probs) return;
     __syncthreads();
-    const Picked o = sh;
-    for (int i = threadIdx.x; i < n; i += kSampleThreads) {
-        const float v = p[i] / o.s;
-        p[i] = top_p < 1.0f && i < o.last ? v / o.z : v;
+    const float s = sh_s;
+    for (int i = tid; i < n; i += kSampleThreads) p[i] = p[i] / s;
+    __syncthreads();
+    int last = n;
+    if (top_p < 1.0f) {
+        if (w0) {
+            const float z = nucleus(n, n, top_p, last, val);
+            if (tid == 0) {
+                sh_z = z;
+                sh_last = last;
+            }
+        }
+        __syncthreads();
+        const float z = sh_z;
+        last = sh_last;
+        for (int i = tid; i < last; i += kSampleThreads) p[i] = p[i] / z;
+        __syncthreads();
+    }
+    if (w0) {
+        const int place = draw(last, r, val);
+        if (tid == 0) *out = idx[place >= 0 ? place : last - 1];
     }
 }
 
@@ -385,8 +408,13 @@ __global__ __launch_bounds__(kSampleThreads) void k_top_sample(const float* logi
         p[i] = expf_libm((logits[(uint32_t)e[i]] - m) / temperature, kExp2Tab);
     __syncthreads();
     if (tid < 64) {
-        const Picked o = pick(p, count, n, top_p, r);
-        const int at = o.place >= 0 ? o.place : o.last - 1;
+        // a division by s or z is the same float wherever it happens: few values, divided as they are read
+        const float s = sum_in_order(count, [&](int i) { return p[i]; });
+        int last = n;
+        float z = 0.0f;
+        if (top_p < 1.0f) z = nucleus(count, n, top_p, last, [&](int i) { return p[i] / s; });
+        const int place = draw(min(count, last), r, [&](int i) { return top_p < 1.0f ? p[i] / s / z : p[i] / s; });
+        const int at = place >= 0 ? place : last - 1;
         // a draw past every sum: the last kept index, the whole order's last one if all are kept
         const unsigned long long lo = wave_max_u64(w->lo[tid]);
         if (tid == 0) *out = (int32_t)(uint32_t)(at < count ? e[at] : lo);
@@ -438,8 +466,7 @@ hipError_t launch_sample(const float* logits, int n, float temperature, float to
     }
     hipLaunchKernelGGL(k_sample_exp, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, logits, idx, p, n,
                        temperature);
-    hipLaunchKernelGGL(k_sample, dim3(1), dim3(kSampleThreads), 0, st, idx, p, n, top_p, r, d_token,
-                       d_probs ? 1 : 0);
+    hipLaunchKernelGGL(k_sample, dim3(1), dim3(kSampleThreads), 0, st, idx, p, n, top_p, r, d_token);
     return hipGetLastError();
 }
 
