@@ -25,8 +25,8 @@
 //
 // Numerics: an fp32 activation is the sum of three bf16 (8 bits each, by truncation, exact
 // with fp32's range, so no row scales), and the block integers of Q8_0, Q4_0 and Q4_1 are exact
-// in bf16: three v_mfma_f32_16x16x32_bf16 give a block's products exactly in the fp32
-// accumulator, and d (and Q4_1's m) scale the block sums in fp32 (quant.cpp:266-321). F16 weights
+// in bf16: every product of three v_mfma_f32_16x16x32_bf16 is exact, their sum over a block is
+// fp32's, and d (and Q4_1's m) scale the block sums in fp32 (quant.cpp:266-321). F16 weights
 // and Q6_K's sc (u - 32) (at most 13 bits) are two bf16, five MFMAs (the dropped third piece
 // times second piece is 2^-24 of the product). rmsnorm's weights multiply the activations before
 // they are split, its row factor the finished sum. (F32 weights would be three pieces, with more
