@@ -17,6 +17,35 @@ namespace gemv_detail {
 constexpr int kStageVec = 9;  // float4 of x per thread
 static_assert(kStageVec * 4 * kBlock == kGemvMaxK, "the row length this prologue holds");
 
+// stage_x's x for rows longer than its registers hold: read twice where it is normalised.
+__device__ void stage_long(const GemvArgs& a, float* xs) {
+    const int K4 = (int)(a.K / 4), tid = threadIdx.x;
+    const float4 *x4 = (const float4*)a.x, *w4 = (const float4*)a.norm_w;
+    float inv = 1.0f;
+    if (w4) {
+        __shared__ double red[kWavesPerBlock];
+        double ss = 0;
+        for (int j = tid; j < K4; j += kBlock) {
+            const float4 v = x4[j];
+            ss += (double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z + (double)v.w * v.w;
+        }
+        ss = wave_sum_d(ss);
+        if ((tid & 63) == 0) red[tid >> 6] = ss;
+        __syncthreads();
+        ss = (red[0] + red[1]) + (red[2] + red[3]);
+        inv = 1.0f / sqrtf((float)(ss / a.K) + a.eps);
+    }
+    for (int j = tid; j < K4; j += kBlock) {
+        float4 v = x4[j];
+        if (w4) {
+            const float4 w = w4[j];
+            v = make_float4(v.x * inv * w.x, v.y * inv * w.y, v.z * inv * w.z, v.w * inv * w.w);
+        }
+        ((float4*)xs)[j] = v;
+        if (a.norm_out && blockIdx.x == 0) ((float4*)a.norm_out)[j] = v;
+    }
+}
+
 // x (optionally RMSNorm-ed) and its 16-element partial sums into LDS. Every load of x
 // and of the norm weight is issued before the first one is used, and the prologue ends
 // with every load complete, the first weight tile's included (issued earlier, it has
@@ -26,51 +55,55 @@ __device__ void stage_x(const GemvArgs& a, float* xs, float* x16, bool need_sums
     const int K4 = (int)(a.K / 4);
     const int nv = (K4 + kBlock - 1) / kBlock;  // float4 of x per thread actually needed
     const int tid = threadIdx.x;
-    const float4* x4 = (const float4*)a.x;
-    // indices past the end re-load the last element (never stored)
-    float4 xv[kStageVec];
-#pragma unroll
-    for (int i = 0; i < kStageVec; ++i) {
-        const int j = tid + i * kBlock;
-        if (i < nv) xv[i] = x4[j < K4 ? j : K4 - 1];
-    }
-    if (a.norm_w) {
-        const float4* w4 = (const float4*)a.norm_w;
-        float4 wv[kStageVec];
+    if (K4 > kStageVec * kBlock) {
+        stage_long(a, xs);
+    } else {
+        const float4* x4 = (const float4*)a.x;
+        // indices past the end re-load the last element (never stored)
+        float4 xv[kStageVec];
 #pragma unroll
         for (int i = 0; i < kStageVec; ++i) {
             const int j = tid + i * kBlock;
-            if (i < nv) wv[i] = w4[j < K4 ? j : K4 - 1];
+            if (i < nv) xv[i] = x4[j < K4 ? j : K4 - 1];
         }
-        __shared__ double red[kWavesPerBlock];
-        double ss = 0;  // every x*x is exact in fp64, as in the reference's accumulation
+        if (a.norm_w) {
+            const float4* w4 = (const float4*)a.norm_w;
+            float4 wv[kStageVec];
 #pragma unroll
-        for (int i = 0; i < kStageVec; ++i) {
-            if (i < nv) {
-                const float4 v = xv[i];
-                const double t = (double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z + (double)v.w * v.w;
-                ss += tid + i * kBlock < K4 ? t : 0.0;
+            for (int i = 0; i < kStageVec; ++i) {
+                const int j = tid + i * kBlock;
+                if (i < nv) wv[i] = w4[j < K4 ? j : K4 - 1];
+            }
+            __shared__ double red[kWavesPerBlock];
+            double ss = 0;  // every x*x is exact in fp64, as in the reference's accumulation
+#pragma unroll
+            for (int i = 0; i < kStageVec; ++i) {
+                if (i < nv) {
+                    const float4 v = xv[i];
+                    const double t = (double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z + (double)v.w * v.w;
+                    ss += tid + i * kBlock < K4 ? t : 0.0;
+                }
+            }
+            ss = wave_sum_d(ss);
+            if ((tid & 63) == 0) red[tid >> 6] = ss;
+            __syncthreads();
+            ss = (red[0] + red[1]) + (red[2] + red[3]);
+            const float inv = 1.0f / sqrtf((float)(ss / a.K) + a.eps);
+#pragma unroll
+            for (int i = 0; i < kStageVec; ++i) {
+                if (i < nv) {
+                    const float4 v = xv[i], w = wv[i];
+                    xv[i] = make_float4(v.x * inv * w.x, v.y * inv * w.y, v.z * inv * w.z, v.w * inv * w.w);
+                }
             }
         }
-        ss = wave_sum_d(ss);
-        if ((tid & 63) == 0) red[tid >> 6] = ss;
-        __syncthreads();
-        ss = (red[0] + red[1]) + (red[2] + red[3]);
-        const float inv = 1.0f / sqrtf((float)(ss / a.K) + a.eps);
 #pragma unroll
         for (int i = 0; i < kStageVec; ++i) {
-            if (i < nv) {
-                const float4 v = xv[i], w = wv[i];
-                xv[i] = make_float4(v.x * inv * w.x, v.y * inv * w.y, v.z * inv * w.z, v.w * inv * w.w);
+            const int j = tid + i * kBlock;
+            if (i < nv && j < K4) {
+                ((float4*)xs)[j] = xv[i];
+                if (a.norm_out && blockIdx.x == 0) ((float4*)a.norm_out)[j] = xv[i];
             }
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < kStageVec; ++i) {
-        const int j = tid + i * kBlock;
-        if (i < nv && j < K4) {
-            ((float4*)xs)[j] = xv[i];
-            if (a.norm_out && blockIdx.x == 0) ((float4*)a.norm_out)[j] = xv[i];
         }
     }
     __syncthreads();

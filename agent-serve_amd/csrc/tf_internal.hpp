@@ -333,7 +333,7 @@ hipError_t launch_step_f16(const StepArgs& a, int n_wg, hipStream_t st);
 hipError_t launch_step_q6k(const StepArgs& a, int n_wg, hipStream_t st);
 
 // Launchers (k_*.hip).
-constexpr int kGemvMaxK = 9216;  // row length launch_gemv's prologue holds (9 float4 a thread)
+constexpr int kGemvMaxK = 9216;  // row length launch_gemv's prologue holds in registers (9 float4 a thread)
 hipError_t launch_gemv(const GemvArgs& a, int rows_per_wave, hipStream_t st);
 int64_t gemv_groups(int64_t n_rows, int rows_per_wave);
 size_t gemv_lds_bytes(int64_t K);

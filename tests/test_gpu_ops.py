@@ -104,6 +104,22 @@ def test_gemv_outlier_blocks(pkg, t, k, n):
         print(f"Q8_0 K={k}: max |gpu - exact| / sum|x w| = {np.max(e / budget):.3e}, median / bound {med:.4f}")
 
 
+@pytest.mark.parametrize("t", [8, 2, 3, 1, 0, 14])
+@pytest.mark.parametrize("k", [9216, 9472, 16384, 20480])
+def test_gemv_long_rows(pkg, t, k):
+    """One row of x against rows up to and past the 9,216 elements that the GEMV's prologue holds in
+    registers, against the exact sums: 23 roundings of a step, K / 1024 of its steps (2^-24 each) of
+    sum |x w|, as in test_gemv_outlier_blocks, times 4 for the formats with an offset term."""
+    rng = np.random.default_rng(k + t)
+    n = 48
+    rows = random_rows(rng, t, k, n)
+    deq = oracle_dequant(t, rows, k).astype(np.float64)
+    x = rng.standard_normal(k).astype(np.float32)
+    got = pkg.matmul(t, rows, k, n, x)[0].astype(np.float64)
+    budget = np.abs(deq) @ np.abs(x).astype(np.float64)
+    assert np.max(np.abs(got - deq @ x.astype(np.float64)) / budget) <= 4 * (24 + k / 1024) * 2.0**-24
+
+
 def test_matmul_several_rows(pkg):
     rng = np.random.default_rng(3)
     k, n = 2048, 256
